@@ -61,6 +61,7 @@ SCRATCH_LIMITS = {
     "dqds128_kernel": 0,
     "decode128_kernel": 0,
     "rmsnorm_kernel": 0,
+    "generic_kernel": 0,
 }
 
 # "Function Name: <kernel>" starts a kernel's block; then "<field> [unit]: value".
