@@ -93,12 +93,15 @@ int lc_attn_fwd_shard(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, 
 
 /* Split-KV decode: the same outputs as lc_attn_fwd_shard for a query shard of
  * a few tokens against a long KV shard (a decode step over a KV cache).  For
- * bf16, head_dim 128 and q_tokens * heads_q / heads_kv <= 16 the key range of
- * each (batch, KV head) is split over many one-wave workgroups that stream the
- * cache, and a second kernel merges the splits by log-sum-exp; it needs a
+ * bf16, head_dim 64 or 128 and q_tokens * heads_q / heads_kv <= 64 the key
+ * range of each (batch, KV head) is split over many waves that stream the
+ * cache, and a second kernel merges what is not merged within a workgroup by
+ * log-sum-exp.  head_dim 128 with q_tokens * heads_q / heads_kv <= 16 needs a
  * 16-byte-aligned workspace of lc_attn_decode_workspace_bytes(shape) bytes
- * (LC_ERR_WORKSPACE if smaller, LC_ERR_INVALID if misaligned).  Other shapes run
- * the lc_attn_fwd_shard kernels (workspace unused; the size query returns 0).
+ * (LC_ERR_WORKSPACE if smaller, LC_ERR_INVALID if misaligned); the other of
+ * these shapes run the lc_attn_fwd_shard kernels when the workspace is
+ * smaller or misaligned, and so do all further shapes (the size query returns
+ * 0 where no workspace is used).
  * No counterpart in the reference, whose generation loops recompute the whole
  * prefill for every new token (src/longctx100m/distributed_infer.py:185-219,
  * rust/longctx100m-model/src/bin/infer.rs:96-106); callers that keep a KV cache
@@ -113,9 +116,10 @@ int lc_attn_decode(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, con
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * split partials live in a file-scope device array of
  * LC_DECODE_STATIC_SCRATCH_BYTES bytes that each GPU the library runs on
- * holds until the process ends; the call allocates nothing.  Shapes whose
- * lc_attn_decode_workspace_bytes exceeds that size are rejected with
- * LC_ERR_WORKSPACE (use lc_attn_decode).  Every call on one GPU shares its
+ * holds until the process ends; the call allocates nothing.  Shapes that need
+ * a workspace and whose lc_attn_decode_workspace_bytes exceeds that size are
+ * rejected with LC_ERR_WORKSPACE (use lc_attn_decode); those that only may use
+ * one run the lc_attn_fwd_shard kernels then.  Every call on one GPU shares its
  * array, so calls that overlap on one GPU (concurrent streams or threads)
  * race; calls ordered on a stream do not.  The array used is that of the
  * stream's device (the current device for a null stream).  Results equal

@@ -59,7 +59,7 @@ SCRATCH_LIMITS = {
     "dq128_kernel": 0,
     "dkdv128_kernel": 64,
     "dqds128_kernel": 0,
-    "decode128_kernel": 0,
+    "decode_kernel": 0,
     "rmsnorm_kernel": 0,
     "generic_kernel": 0,
 }

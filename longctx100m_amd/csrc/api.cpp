@@ -392,12 +392,17 @@ int lc_attn_decode(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, con
       !aligned16(o))
     return fwd_shard(p, q, k, v, o, m, l, st);  // the blockwise kernels, no workspace
   const size_t need = round_up(lc::decode_workspace_bytes(p));
-  if (workspace == nullptr || workspace_bytes < need)
+  const bool fits = need == 0 || (workspace != nullptr && workspace_bytes >= need);
+  if (!lc::decode_workspace_required(p)) {
+    // Shapes that once took no workspace: without a usable one, the blockwise kernels.
+    if (!fits || (need > 0 && !aligned16(workspace))) return fwd_shard(p, q, k, v, o, m, l, st);
+  } else if (!fits) {
     return set_error(LC_ERR_WORKSPACE, "decode workspace of %zu bytes is smaller than %zu",
                      workspace_bytes, need);
-  if (!aligned16(workspace))  // the split kernel stores 16-byte vectors of partials
+  } else if (!aligned16(workspace)) {  // the split kernel stores 16-byte vectors of partials
     return set_error(LC_ERR_INVALID, "decode workspace must be 16-byte aligned");
-  hipError_t e = lc::launch_decode128(p, q, k, v, o, m, l, workspace, st);
+  }
+  hipError_t e = lc::launch_decode(p, q, k, v, o, m, l, workspace, st);
   return e == hipSuccess ? LC_OK : hip_error(e, "lc_attn_decode launch");
 }
 
@@ -421,6 +426,26 @@ int lc_attn_decode_static(const lc_attn_shape_t* shape, const lc_attn_mask_t* ma
       !aligned16(o))
     return fwd_shard(p, q, k, v, o, m, l, st);  // the blockwise kernels use no scratch
   const size_t need = round_up(lc::decode_workspace_bytes(p));
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
+  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
+    return fwd_shard(p, q, k, v, o, m, l, st);
   if (need > lc::kDecodeStaticScratchBytes)
     return set_error(LC_ERR_WORKSPACE,
                      "decode needs %zu bytes of scratch, more than the static maximum of %zu; "
@@ -428,7 +453,7 @@ int lc_attn_decode_static(const lc_attn_shape_t* shape, const lc_attn_mask_t* ma
                      need, lc::kDecodeStaticScratchBytes);
   void* scratch = nullptr;
   LC_TRY_HIP(lc::decode_static_scratch(st, &scratch), "lc_attn_decode_static scratch address");
-  hipError_t e = lc::launch_decode128(p, q, k, v, o, m, l, scratch, st);
+  hipError_t e = lc::launch_decode(p, q, k, v, o, m, l, scratch, st);
   return e == hipSuccess ? LC_OK : hip_error(e, "lc_attn_decode_static launch");
 }
 

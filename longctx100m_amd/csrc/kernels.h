@@ -96,12 +96,18 @@ hipError_t launch_bwd_preprocess(int B, int N, int H, int D, int dtype, const vo
                                  const void* dout, const float* m, const float* l, float* delta,
                                  float* lse2, hipStream_t s);
 
-// Split-KV decode attention (decode.hip): bf16, D = 128, Nq * Hq / Hkv <= 16.
+// Split-KV decode attention (decode.hip): bf16, D = 64 or 128, at most
+// kDecodeMaxRows query rows (Nq * Hq / Hkv) per KV head.
+// decode_workspace_required: a workspace of decode_workspace_bytes must be
+// given (D = 128, at most 16 rows); other shapes may run the blockwise kernels
+// instead, and need none when decode_workspace_bytes is 0.
+constexpr int64_t kDecodeMaxRows = 64;
 bool decode_supported(const Problem& p);
+bool decode_workspace_required(const Problem& p);
 int decode_splits(const Problem& p);
 size_t decode_workspace_bytes(const Problem& p);
-hipError_t launch_decode128(const Problem& p, const void* q, const void* k, const void* v,
-                            float* o, float* m, float* l, void* ws, hipStream_t s);
+hipError_t launch_decode(const Problem& p, const void* q, const void* k, const void* v, float* o,
+                         float* m, float* l, void* ws, hipStream_t s);
 // Bytes of decode.hip's file-scope device array that stands in for the
 // workspace of lc_attn_decode_static, and that array's address on the
 // device of stream st (the current device for a null stream; looked up once
