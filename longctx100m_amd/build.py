@@ -55,6 +55,9 @@ EXTRA_FLAGS = {
 # dK/dV kernel keeps a few loop-invariant mask values in scratch, reloaded only
 # on tiles that need the mask.
 SCRATCH_LIMITS = {
+    "fwd64_kernel": 0,
+    "dq64_kernel": 0,
+    "dkdv64_kernel": 0,
     "fwd128_kernel": 0,
     "dq128_kernel": 0,
     "dkdv128_kernel": 64,

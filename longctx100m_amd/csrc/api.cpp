@@ -143,7 +143,7 @@ int fwd_shard(const lc::Problem& p, const void* q, const void* k, const void* v,
       }
     }
   } else if (use_mfma(p, q, k, v, nullptr)) {
-    e = lc::launch_fwd_mfma(p, q, k, v, o, m, l, st);
+    e = lc::launch_fwd64(p, q, k, v, o, m, l, st);
   } else {
     e = lc::launch_fwd_generic(p, q, k, v, o, m, l, st);
   }
@@ -161,7 +161,7 @@ int bwd_shard(const lc::Problem& p, const void* q, const void* k, const void* v,
     if (!mf) {
       e = lc::launch_bwd_dq_generic(p, q, k, v, dout, lse2, delta, dq, st);
     } else if (!d128) {
-      e = lc::launch_bwd_dq_mfma(p, q, k, v, dout, lse2, delta, dq, st);
+      e = lc::launch_dq64(p, q, k, v, dout, lse2, delta, dq, st);
     } else if (p.Nk <= kStreamChunk) {
       e = lc::launch_dq128(p, q, k, v, dout, lse2, delta, dq, st);
     } else {  // key sub-shards
@@ -183,7 +183,7 @@ int bwd_shard(const lc::Problem& p, const void* q, const void* k, const void* v,
     if (!mf) {
       e = lc::launch_bwd_dkdv_generic(p, q, k, v, dout, lse2, delta, dk, dv, st);
     } else if (!d128) {
-      e = lc::launch_bwd_dkdv_mfma(p, q, k, v, dout, lse2, delta, dk, dv, st);
+      e = lc::launch_dkdv64(p, q, k, v, dout, lse2, delta, dk, dv, st);
     } else if (p.Nq <= kStreamChunk) {
       e = lc::launch_dkdv128(p, q, k, v, dout, lse2, delta, dk, dv, st);
     } else {  // query sub-shards

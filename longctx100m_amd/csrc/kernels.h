@@ -39,7 +39,7 @@ bool mfma_supported(const Problem& p);
 // key, p.Nk and p.k_pos0 describe the sub-shard, kv_rows is the key count of
 // the whole shard (the batch stride of K and V; -1: p.Nk), and accumulate
 // merges the result into the running (o, m, l) with the weights of
-// lc_attn_merge instead of overwriting them (launch_fwd_mfma and
+// lc_attn_merge instead of overwriting them (launch_fwd64 and
 // launch_fwd_generic take it from p.accumulate).
 hipError_t launch_fwd128(const Problem& p, const void* q, const void* k, const void* v, float* o,
                          float* m, float* l, hipStream_t s, int64_t kv_rows = -1,
@@ -65,18 +65,18 @@ hipError_t launch_dqds128(const Problem& p, const void* k, const uint16_t* ds, i
                           int ds_nkb, float* dq, hipStream_t s, int64_t k_rows = -1,
                           int64_t q_rows = -1);
 
-// head_dim 64 (and 128 on request): register-staged tiles (fwd_mfma.hip, bwd_mfma.hip).
-hipError_t launch_fwd_mfma(const Problem& p, const void* q, const void* k, const void* v, float* o,
-                           float* m, float* l, hipStream_t s);
+// head_dim 64 (attn64.hip).
+hipError_t launch_fwd64(const Problem& p, const void* q, const void* k, const void* v, float* o,
+                        float* m, float* l, hipStream_t s);
+hipError_t launch_dq64(const Problem& p, const void* q, const void* k, const void* v,
+                       const void* dout, const float* lse2, const float* delta, float* dq,
+                       hipStream_t s);
+hipError_t launch_dkdv64(const Problem& p, const void* q, const void* k, const void* v,
+                         const void* dout, const float* lse2, const float* delta, float* dk,
+                         float* dv, hipStream_t s);
 hipError_t launch_fwd_generic(const Problem& p, const void* q, const void* k, const void* v,
                               float* o, float* m, float* l, hipStream_t s);
 
-hipError_t launch_bwd_dq_mfma(const Problem& p, const void* q, const void* k, const void* v,
-                              const void* dout, const float* lse2, const float* delta, float* dq,
-                              hipStream_t s);
-hipError_t launch_bwd_dkdv_mfma(const Problem& p, const void* q, const void* k, const void* v,
-                                const void* dout, const float* lse2, const float* delta, float* dk,
-                                float* dv, hipStream_t s);
 hipError_t launch_bwd_dq_generic(const Problem& p, const void* q, const void* k, const void* v,
                                  const void* dout, const float* lse2, const float* delta,
                                  float* dq, hipStream_t s);

@@ -109,6 +109,13 @@ __device__ __forceinline__ void dma_b32(const void* base, uint32_t off, uint32_t
                : "memory");
 }
 
+__device__ __forceinline__ void dma_b32(const void* g, uint32_t lds) {
+  asm volatile("s_nop 4\n\tglobal_load_lds_dword %0, off"
+               :
+               : "v"(g), "{m0}"(__builtin_amdgcn_readfirstlane(lds))
+               : "memory");
+}
+
 // Direct global->LDS loader for tiles of ROWS rows of a [*, 128] bf16
 // matrix (row stride `stride` elements), NW waves, one wave instruction per
 // 4 rows.  The per-lane byte offsets inside a tile and the wave's LDS offset
