@@ -24,15 +24,16 @@
 // takes 2 us to arrive, a workgroup 1 us to start.  Measured against the
 // blockwise forward that head_dim 64 and more than 16 rows took before (one
 // query call, caches cold): 4 sequences x 3,001 keys, 9/3 heads of 64
-// 69.9 -> 8.8 us; 8 tokens x 32/8 heads of 128 over 16,001 keys 266 -> 22.4 us;
-// 16 sequences x 60,000 keys of the same 1310 -> 699 us.  Against one-wave
+// 69.9 -> 9.0 us; 8 tokens x 32/8 heads of 128 over 16,001 keys 266 -> 22.3 us;
+// 16 sequences x 60,000 keys of the same 1310 -> 730 us.  Against one-wave
 // workgroups with a merge for every shape: 8,001 keys x 32/8 heads
-// 15.2 -> 12.6 us, 16 x 4,000 66.7 -> 52.8 us.
+// 15.2 -> 12.9 us, 16 x 4,000 66.7 -> 53 us.
 #include "common.h"
 #include "kernels.h"
 #include "tile128.h"
 
 #include <algorithm>
+#include <cstdint>
 #include <mutex>
 #include <type_traits>
 
@@ -482,43 +483,42 @@ int64_t row_blocks(const Problem& p) {
 // of 4,000 keys 52.7 / 55.9 / 82.4.  A long single stream is the exception:
 // one-wave workgroups put the same keys of up to eight KV heads, adjacent in
 // memory, on one CU, which reads 262,144 keys x 8 heads at 6.4 against 5.5
-// TB/s (1,000,000 x 16 at 6.2 against 5.7).
+// TB/s (1,000,000 x 16 at 6.2 against 5.7; 60,000 x 8 in 45 us against 46).
 int waves_for(const Problem& p) {
   const int64_t units = (int64_t)p.B * p.Hkv * row_blocks(p);
   const int64_t tiles = (int64_t)p.Nk * p.D * 2 / kTileBytes;
-  return units <= 16 && tiles * units >= 8 * kWaveSlots ? kStreamWaves : kWaves;
+  return units <= 16 && tiles * units >= 6 * kWaveSlots ? kStreamWaves : kWaves;
 }
 
-// Workgroups per (batch, KV head, row block): the count with the least
-// estimated time.  A workgroup takes a few microseconds to start and end and
-// then a tile time per tile of its waves, which is the latency of a tile
-// while few workgroups run and the memory rate once all do; a second kernel
-// merges more than one split.
+// Workgroups per (batch, KV head, row block).  A workgroup saturates its CU's
+// share of the memory, so their number should be just below a multiple of the
+// 256 CUs: the S for up to four per CU that takes the fewest tile steps, a
+// start counting as one (8 KV heads: 8,000 keys 13.0 us with 32 splits against
+// 14.8 with 48 and 16.4 with 16, 24,000 keys 23.8 / 26.4 / 26.6; 14 KV heads x
+// 20,000 keys 30.8 us with 224 workgroups against 41.2 with 266).  Once every
+// wave would walk twelve tiles eight per CU even out the CUs' rates (64 KV
+// heads x 50,000 keys of 64 135 us against 150 with four, 256 heads x 60,000
+// 1.22 ms against 1.33); short caches take a tile per wave (4,000 keys 9.8 us
+// against 11.6 at two), and up to four tiles a wave one workgroup is as fast as
+// the merge it saves (500 keys: 7.8 us against 7.6; 300 keys 6.4 against 8.1).
 int choose_splits(const Problem& p) {
-  constexpr double kStart = 4.0, kTileLatency = 2.2, kTileFull = 5.2, kMerge = 4.5;  // us
   const int64_t units = (int64_t)p.B * p.Hkv * row_blocks(p);
   const int tk = kTileBytes / (2 * p.D);
-  const int64_t tiles = ((int64_t)p.Nk + tk - 1) / tk;
-  const int64_t waves = waves_for(p), slots = kWaveSlots / waves;
-  int best = 1;
-  double best_us = 0;
-  auto consider = [&](int64_t s) {
-    s = std::max<int64_t>(1, std::min<int64_t>(s, kMaxSplits));
-    if (s > 1 && (s - 1) * waves >= tiles) return;  // a workgroup without keys
-    const int64_t wgs = units * s, rounds = (wgs + slots - 1) / slots;
-    const double per_wave = double((tiles + s * waves - 1) / (s * waves));
-    const double fill = double(std::min(wgs, slots)) / double(slots);
-    const double us = double(rounds) * (kStart + per_wave * std::max(kTileLatency, kTileFull * fill)) +
-                      (s > 1 ? kMerge + 0.02 * double(s) : 0.0);
-    if (best_us == 0 || us < best_us) {
-      best = (int)s;
-      best_us = us;
+  const int64_t tiles = ((int64_t)p.Nk + tk - 1) / tk, waves = waves_for(p);
+  const int64_t most = std::min<int64_t>((tiles + waves - 1) / waves, kMaxSplits);
+  if (tiles <= 4 * waves) return 1;
+  if (waves == kStreamWaves) return (int)std::min((kWaveSlots + units - 1) / units, most);
+  int64_t best = 1, best_steps = INT64_MAX;
+  for (int64_t k = 1; k <= 4; ++k) {
+    const int64_t s = std::min(std::max<int64_t>(1, 256 * k / units), most);
+    const int64_t steps = ((units * s + 255) / 256) * ((tiles + s * waves - 1) / (s * waves) + 1);
+    if (steps < best_steps) {
+      best = s;
+      best_steps = steps;
     }
-  };
-  consider(1);
-  for (int64_t fill = slots; fill <= 4 * slots; fill *= 2) consider(fill / units);  // whole rounds
-  for (int64_t t = 1; t <= 4; t *= 2) consider((tiles + waves * t - 1) / (waves * t));  // t tiles a wave
-  return best;
+  }
+  if (tiles >= 12 * waves * best) best = std::min(std::max(best, kWaveSlots / units), most);
+  return (int)best;
 }
 
 size_t partial_bytes(const Problem& p, int64_t S) {
