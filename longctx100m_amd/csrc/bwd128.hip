@@ -14,7 +14,8 @@
 //           tiles of K and V double-buffered in LDS.
 //             S^T = K Q^T, dP^T = V dO^T   (A = K, V rows: ds_read_b128)
 //             dQ^T += K^T dS^T             (A = K^T: ds_read_b64_tr_b16)
-//   dkdv128 KV-stationary, 4 waves x 32 keys of one KV head, walking every
+//   dkdv128 KV-stationary, 4 waves x 32 keys of one KV head (small grids: 2 key
+//           waves in each of 4 groups that split the walk), walking every
 //           query head of the GQA group (group sum in registers).  K^T in
 //           VGPRs, the workgroup's V rows in LDS (negated once, so that
 //           the dP accumulator runs from delta to delta - dP); 32-query
@@ -302,9 +303,6 @@ __global__ __launch_bounds__(256, 2) void dq128_kernel(Bwd128Args a) {
 // every query of the wave) is replaced by zeros; inside a written block every
 // masked score already has dS = 0.
 constexpr int kDsWaveBytes = 2 * 2 * kDsBlockElems;  // a wave's two blocks of one tile
-constexpr int kDsStages = 2;  // dS tiles in LDS: the one in use and one in flight
-constexpr int kDsNW = 16;     // waves per workgroup (4 per SIMD: <= 128 VGPRs)
-constexpr int kDsBM = kDsNW * kDqQW;  // queries per workgroup
 
 __device__ __forceinline__ int ds_query(int j) {
   const int c = j & 15, cb = j >> 4;
@@ -313,7 +311,11 @@ __device__ __forceinline__ int ds_query(int j) {
 
 // LDS: K double-buffered and dS in kDsStages buffers, both one tile ahead (the
 // dS stream comes from HBM): 160 KB, one workgroup per CU.
+template <int kDsNW>
 __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
+  constexpr int kDsBM = kDsNW * kDqQW;  // queries per workgroup
+  // dS tiles in LDS: the one in use and one in flight, two with few waves.
+  constexpr int kDsStages = kDsNW == 4 ? 3 : 2;
   __shared__ __attribute__((aligned(1024))) uint8_t kbuf[2][kDqTile];
   __shared__ __attribute__((aligned(1024))) uint8_t dsbuf[kDsStages][kDsNW][kDsWaveBytes];
 
@@ -374,6 +376,7 @@ __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
   };
   ld.load(kbase, ks, 0, a.Nk, kbuf_lds, wave, lane);
   load_ds(0);
+  if constexpr (kDsStages == 3) load_ds(1);
 
   // B operand read of k-step 0, k-half 0: lane (group G, index i) addresses
   // row key(hh, 0, t) of half G % 2, chunk g = i % 4 (u = g / 2, byte 8 (g % 2)).
@@ -390,11 +393,13 @@ __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
   for (int i = 0; i < 4; ++i) acc[i] = f32x16{};
 
   for (int j = 0; j < ntiles; ++j) {
-    t128::wait_vmem();  // K_j and dS_j
+    // K_j and dS_j, not dS_{j+1}, whose four loads were issued after them
+    if (kDsStages == 3 && j + 1 < nt_w) t128::wait_vmem_but<4>();
+    else t128::wait_vmem();
     __syncthreads();
     if (j + 1 < ntiles)
       ld.load(kbase, ks, (j + 1) * kDqBN, a.Nk, kbuf_lds + ((j + 1) & 1) * kDqTile, wave, lane);
-    load_ds(j + 1);
+    load_ds(j + kDsStages - 1);
     if (j >= nt_w) continue;
     const uint8_t* kt = kbuf[j & 1];
     const uint8_t* dt = dsbuf[j % kDsStages][wave];
@@ -443,8 +448,8 @@ __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
 // ---------------------------------------------------------------- dK/dV --
 
 constexpr int kKvKW = 32;
-constexpr int kKvBN = 4 * kKvKW;  // keys per workgroup
-constexpr int kKvBM = 32;         // queries per tile
+constexpr int kKvBM = 32;             // queries per tile
+constexpr int kPartPitch = D + 4;     // floats per key of a group's partial
 constexpr int kKvTile = kKvBM * t128::kRowBytes;
 
 // dK/dV with v_mfma_f32_32x32x16_bf16: one 32x32 score block per wave and
@@ -456,14 +461,23 @@ constexpr int kKvTile = kKvBM * t128::kRowBytes;
 // Score element v of lane l: query 8(v/4) + 4(l/32) + v%4, key l%32.  As a B
 // operand, k-step u (queries 16u .. 16u+15) takes, in slot 4p + t, element
 // 8u + 4(t/2) + 2(t%2) + p, i.e. query 16u + row(h, p, t) of tr32_off.
-__global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[2][2][kKvTile];  // [buf][Q,dO]
-  __shared__ __attribute__((aligned(1024))) uint8_t v_lds[kKvBN * t128::kRowBytes];
-  __shared__ __attribute__((aligned(16))) float stat[2][2][64];           // [buf][lse2,delta]
+template <int KW, int QS>
+__global__ __launch_bounds__(64 * KW * QS, 2) void dkdv128_kernel(Bwd128Args a) {
+  constexpr int kKvBN = KW * kKvKW;       // keys per workgroup
+  constexpr int kGroupLds = 4 * kKvTile;  // a group's tiles: [buf][Q, dO]
+  constexpr int kVBytes = kKvBN * t128::kRowBytes;
+  // V rows, then each group's tiles; after the walk the partials of the groups.
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kVBytes + QS * kGroupLds];
+  __shared__ __attribute__((aligned(16))) float stat[QS][2][2][64];  // [group][buf][lse2,delta]
+  const uint8_t* v_lds = smem;
+  static_assert(QS == 1 || KW * QS * kKvKW * kPartPitch * 4 <= kVBytes + QS * kGroupLds,
+                "one accumulator's partials fit");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave_wg = QS == 1 ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = QS == 1 ? wave_wg : wave_wg % KW;  // among the group's
+  const int grp = QS == 1 ? 0 : wave_wg / KW;
   const int kc = lane & 31;  // key column of the wave's 32 keys
   const int h = lane >> 5;
 
@@ -493,20 +507,29 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
   const int ntq = any_valid_key ? (a.Nq - qstart + kKvBM - 1) / kKvBM : 0;
   const int nsteps = ntq * a.group;
   if (nsteps == 0) return;  // no visible (query, key) pair: no contribution
+  // Group g takes the steps g, g + QS, ...; every group passes every barrier.
+  const int niter = QS == 1 ? nsteps : (nsteps + QS - 1) / QS;
 
-  t128::RowLoader<kKvBM, 4> ld;
+  t128::RowLoader<kKvBM, KW> ld;
   ld.init(qs, wave, lane);
+  const uint32_t tiles_lds = t128::lds_addr(smem) + kVBytes + grp * kGroupLds;
+  const uint32_t stat_lds = t128::lds_addr(stat) + grp * 1024;
   auto issue = [&](int hq, int qrow0, int buf) {
     const uint16_t* qb = a.q + (int64_t)b * a.q_rows * qs + (int64_t)hq * D;
     const uint16_t* ob = a.dout + (int64_t)b * a.q_rows * qs + (int64_t)hq * D;
-    ld.load(qb, qs, qrow0, a.Nq, t128::lds_addr(smem) + buf * 2 * kKvTile, wave, lane);
-    ld.load(ob, qs, qrow0, a.Nq, t128::lds_addr(smem) + (buf * 2 + 1) * kKvTile, wave, lane);
+    ld.load(qb, qs, qrow0, a.Nq, tiles_lds + buf * 2 * kKvTile, wave, lane);
+    ld.load(ob, qs, qrow0, a.Nq, tiles_lds + (buf * 2 + 1) * kKvTile, wave, lane);
     const int64_t sbase = ((int64_t)b * a.Hq + hq) * a.q_rows;
-    if (wave == 0) t128::load_f32x64(a.lse2 + sbase, qrow0, a.Nq, t128::lds_addr(stat) + buf * 512, lane);
-    if (wave == 1) t128::load_f32x64(a.delta + sbase, qrow0, a.Nq, t128::lds_addr(stat) + buf * 512 + 256, lane);
+    if (wave == 0) t128::load_f32x64(a.lse2 + sbase, qrow0, a.Nq, stat_lds + buf * 512, lane);
+    if (wave == 1) t128::load_f32x64(a.delta + sbase, qrow0, a.Nq, stat_lds + buf * 512 + 256, lane);
   };
-  const int hq0 = hk * a.group;
-  issue(hq0, qstart, 0);
+  // The group's first step: (head, query tile) number grp of the walk.
+  int hq0 = hk * a.group, qfirst = qstart;
+  if constexpr (QS > 1) {
+    hq0 += grp / ntq;
+    qfirst += grp % ntq * kKvBM;
+  }
+  if (QS == 1 || grp < nsteps) issue(hq0, qfirst, 0);
 
   // K^T as the B operand in VGPRs: lane l holds key kw0 + l%32, dims 16t + 8h .. +7.
   bf16x8 kreg[D / 16];
@@ -517,9 +540,9 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
       kreg[t] = *reinterpret_cast<const bf16x8*>(kbase + (int64_t)row * ks + 16 * t + 8 * h);
   }
   {
-    t128::RowLoader<kKvBN, 4> vld;
-    vld.init(ks, wave, lane);
-    vld.load(vbase, ks, k0, a.Nk, t128::lds_addr(v_lds), wave, lane);
+    t128::RowLoader<kKvBN, KW * QS> vld;
+    vld.init(ks, wave_wg, lane);
+    vld.load(vbase, ks, k0, a.Nk, t128::lds_addr(smem), wave_wg, lane);
   }
   // K^T is in VGPRs from here on.  Without this wait the compiler (which
   // cannot tell how many vector memory operations the loop's waits leave
@@ -528,13 +551,16 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
   t128::wait_vmem();
   // V enters dP = dO V^T negated, so that the dP accumulator can start at
   // delta and end at delta - dP: dS = P (dP - delta) = -(P (delta - dP)).
-  // Each wave negates the 32 rows it reads (written by every wave's DMA).
+  // Each wave negates its share of the rows (written by every wave's DMA); with
+  // one group those are the rows it reads itself, otherwise the first step's
+  // barrier comes between.
   __syncthreads();
   {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    uint8_t* vw = v_lds + wave * kKvKW * t128::kRowBytes + lane * 16;
+    constexpr int kShare = kVBytes / (KW * QS);
+    uint8_t* vw = smem + wave_wg * kShare + lane * 16;
 #pragma unroll
-    for (int i = 0; i < kKvKW * t128::kRowBytes / 1024; ++i) {
+    for (int i = 0; i < kShare / 1024; ++i) {
       u32x4* p = reinterpret_cast<u32x4*>(vw + i * 1024);
       *p = *p ^ 0x80008000u;
     }
@@ -563,15 +589,18 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
   // MFMAs: the V tile holds -V, so E ends at delta - dP (one multiply per
   // element instead of a subtraction and a multiply).
   bf16x8 ds_keep[2];  // the last tile's packed dS (both k-steps), stored at the next step's top
-  auto tile = [&](auto masked_tag, int buf, int cthr, int kmax, int qmax) {
-    constexpr bool MASKED = decltype(masked_tag)::value;
-    const uint8_t* qt_ = &smem[0][0][0];
-    const uint8_t* ot_ = &smem[0][1][0];
-    const float* lse_ = stat[buf][0];
-    const float* dlt_ = stat[buf][1];
+  // masked: a std::bool_constant (an instantiation each; the one-group kernel,
+  // whose registers just suffice) or a uniform bool (one instantiation, fewer
+  // registers; with groups two of them spill).
+  auto tile = [&](auto masked, int buf, int cthr, int kmax, int qmax) {
+    constexpr bool STATIC = !std::is_same<decltype(masked), bool>::value;
+    const uint8_t* qt_ = smem + kVBytes;
+    const uint8_t* ot_ = smem + kVBytes + kKvTile;
+    const float* lse_ = stat[grp][buf][0];
+    const float* dlt_ = stat[grp][buf][1];
     // The buffer offset (a multiple of 16 KB) is folded into the per-lane
     // bases: the swizzle XORs change only bits 5-7 of an offset below 8 KB.
-    const int bo = buf * 2 * kKvTile;
+    const int bo = grp * kGroupLds + buf * 2 * kKvTile;
     const int ro = opaque(roff0 + bo), vo = opaque(voff0);
     const int to0 = opaque(toff0 + bo), to1 = opaque(toff1 + bo);
     auto ld = [](const uint8_t* p) { return *reinterpret_cast<const bf16x8*>(p); };
@@ -591,11 +620,13 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
     };
     int kq = 0, qlim = 0;
     bool kbad = false;
-    if constexpr (MASKED) {
+    if (masked) {
       kq = opaque(kc - 4 * h);
       qlim = opaque(qmax - 4 * h);
       kbad = kc >= kmax;
     }
+    // query 4h + qo of the tile against key kc: the per-lane parts are kq, qlim
+    auto hidden = [&](int qo) { return kbad || (a.causal && kq > cthr + qo) || qo >= qlim; };
     f32x16 sv, dpv, dinit;
     bf16x8 A[2], B[2], pb[2], db[2];
     f32x4 st[2];  // lse2 quads, loaded two steps before use
@@ -630,6 +661,12 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
           for (int r = 0; r < 4; ++r) dinit[4 * w + r] = d4[r];
         }
       }
+      if constexpr (!STATIC) {
+        if (j == 8 && masked) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) sv[v] = hidden(8 * (v >> 2) + (v & 3)) ? -INFINITY : sv[v];
+        }
+      }
       // P for elements 2k, 2k+1 at j = 9 + k
       if (j >= 9 && j <= 16) {
         const int k = j - 9;
@@ -637,11 +674,8 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
         for (int e = 0; e < 2; ++e) {
           const int v = 2 * k + e, w = v >> 2, r = v & 3;
           float x = sv[v];
-          if constexpr (MASKED) {
-            // query 4h + (8w + r) against key kc: the per-lane parts are kq, qlim
-            const int qo = 8 * w + r;
-            const bool bad = kbad || (a.causal && kq > cthr + qo) || qo >= qlim;
-            x = bad ? -INFINITY : x;
+          if constexpr (STATIC) {
+            if (masked) x = hidden(8 * w + r) ? -INFINITY : x;
           }
           sv[v] = fast_exp2(fmaf(x, a.sl2, -st[w & 1][r]));
         }
@@ -676,8 +710,22 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
     }
   };
 
-  int cur_q = qstart, cur_hq = hq0;    // step being computed
-  int nxt_hq = hq0, nxt_q = qstart;    // step being prefetched
+  int cur_q = qfirst, cur_hq = hq0;    // step being computed
+  int nxt_hq = hq0, nxt_q = qfirst;    // step being prefetched
+  auto advance = [&](int& q, int& hq) {
+    q += QS * kKvBM;
+    if constexpr (QS == 1) {
+      if (q >= a.Nq) {
+        q = qstart;
+        ++hq;
+      }
+    } else {
+      while (q >= qstart + ntq * kKvBM) {
+        q -= ntq * kKvBM;
+        ++hq;
+      }
+    }
+  };
   // dS stores: a tile's dS is stored at the top of the next step, after that
   // step's tile loads, so the wait for those loads at the following top does
   // not include the stores (vector memory operations complete in issue order,
@@ -691,30 +739,23 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
     __builtin_nontemporal_store(ds_keep[0], (gbl_bf16x8*)(blk + 16 * dsl));
     __builtin_nontemporal_store(ds_keep[1], (gbl_bf16x8*)(blk + 1024 + 16 * (dsl ^ 8)));
   };
-  for (int step = 0; step < nsteps; ++step) {
+  for (int step = 0; step < niter; ++step) {
     if (stored)
       t128::wait_vmem_but<2>();  // the tile loads, not the stores issued after them
     else
       t128::wait_vmem();
     __syncthreads();
     stored = false;
-    nxt_q += kKvBM;
-    if (nxt_q >= a.Nq) {
-      nxt_q = qstart;
-      ++nxt_hq;
-    }
-    if (step + 1 < nsteps) issue(nxt_hq, nxt_q, (step + 1) & 1);
+    advance(nxt_q, nxt_hq);
+    if ((step + 1) * QS + grp < nsteps) issue(nxt_hq, nxt_q, (step + 1) & 1);
     if (pend >= 0) {  // the previous tile's dS, after the loads
       store_ds(pend);
       stored = true;
       pend = -1;
     }
     const int qrow0 = cur_q, hq_c = cur_hq;
-    cur_q += kKvBM;
-    if (cur_q >= a.Nq) {
-      cur_q = qstart;
-      ++cur_hq;
-    }
+    advance(cur_q, cur_hq);
+    if (QS > 1 && step * QS + grp >= nsteps) continue;
     const int64_t qp_first = a.q_pos0 + qrow0;
     const int64_t qp_last = qp_first + kKvBM - 1;
     if (kw0 >= a.Nk) continue;
@@ -723,36 +764,67 @@ __global__ __launch_bounds__(256, 2) void dkdv128_kernel(Bwd128Args a) {
     const int64_t dsblk = a.ds == nullptr ? -1
         : (((int64_t)b * a.Hq + hq_c) * a.ds_nqt + qrow0 / kKvBM) * a.ds_nkb + kw0 / kKvKW;
     pend = dsblk;
-    if ((a.causal && wk_last > qp_first) || wk_last >= a.valid || kw0 + kKvKW > a.Nk ||
-        qrow0 + kKvBM > a.Nq) {
-      const int64_t ct = qp_first - wk_first;
-      const int cthr = (int)(ct < -4096 ? -4096 : (ct > 4096 ? 4096 : ct));
-      const int64_t km = min((int64_t)(a.Nk - kw0), a.valid - wk_first);
-      const int kmax = (int)(km < 0 ? 0 : (km > kKvKW ? kKvKW : km));
-      const int qmax = min(a.Nq - qrow0, kKvBM);
-      tile(std::true_type{}, buf, cthr, kmax, qmax);
+    const bool masked = (a.causal && wk_last > qp_first) || wk_last >= a.valid ||
+                        kw0 + kKvKW > a.Nk || qrow0 + kKvBM > a.Nq;
+    const int64_t ct = qp_first - wk_first;
+    const int cthr = (int)(ct < -4096 ? -4096 : (ct > 4096 ? 4096 : ct));
+    const int64_t km = min((int64_t)(a.Nk - kw0), a.valid - wk_first);
+    const int kmax = (int)(km < 0 ? 0 : (km > kKvKW ? kKvKW : km));
+    const int qmax = min(a.Nq - qrow0, kKvBM);
+    if constexpr (QS > 1) {
+      tile(masked, buf, cthr, kmax, qmax);
     } else {
-      tile(std::false_type{}, buf, 0, kKvKW, kKvBM);
+      if (masked) tile(std::true_type{}, buf, cthr, kmax, qmax);
+      else tile(std::false_type{}, buf, 0, kKvKW, kKvBM);
     }
   }
   if (pend >= 0) store_ds(pend);
 
   // dK^T / dV^T element v of lane l: key kw0 + l%32, dim 32*dblk + 8(v/4) + 4h + v%4.
-  const int row = kw0 + kc;
-  if (row < a.Nk) {
-    const int64_t off = (((int64_t)b * a.k_rows + row) * a.Hkv + hk) * D;
+  if constexpr (QS == 1) {
+    const int row = kw0 + kc;
+    if (row < a.Nk) {
+      const int64_t off = (((int64_t)b * a.k_rows + row) * a.Hkv + hk) * D;
 #pragma unroll
-    for (int dblk = 0; dblk < 4; ++dblk)
+      for (int dblk = 0; dblk < 4; ++dblk)
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const int d0 = 32 * dblk + 8 * w + 4 * h;
-        f32x4* pk = reinterpret_cast<f32x4*>(a.dk + off + d0);
-        f32x4* pv = reinterpret_cast<f32x4*>(a.dv + off + d0);
-        const f32x4 k4 = {dk[dblk][4 * w], dk[dblk][4 * w + 1], dk[dblk][4 * w + 2], dk[dblk][4 * w + 3]};
-        const f32x4 v4 = {dv[dblk][4 * w], dv[dblk][4 * w + 1], dv[dblk][4 * w + 2], dv[dblk][4 * w + 3]};
-        *pk = *pk + k4 * a.scale;
-        *pv = *pv + v4;
+        for (int w = 0; w < 4; ++w) {
+          const int d0 = 32 * dblk + 8 * w + 4 * h;
+          f32x4* pk = reinterpret_cast<f32x4*>(a.dk + off + d0);
+          f32x4* pv = reinterpret_cast<f32x4*>(a.dv + off + d0);
+          const f32x4 k4 = {dk[dblk][4 * w], dk[dblk][4 * w + 1], dk[dblk][4 * w + 2], dk[dblk][4 * w + 3]};
+          const f32x4 v4 = {dv[dblk][4 * w], dv[dblk][4 * w + 1], dv[dblk][4 * w + 2], dv[dblk][4 * w + 3]};
+          *pk = *pk + k4 * a.scale;
+          *pv = *pv + v4;
+        }
+    }
+  } else {
+    // The groups' partials meet in LDS, dK first, then dV.
+    float* part = reinterpret_cast<float*>(smem);
+    auto reduce = [&](const f32x16 (&acc)[4], float* out, float scale) {
+      __syncthreads();  // the tiles, or the previous partials, are done with
+      float* prow = part + (wave_wg * kKvKW + kc) * kPartPitch + 4 * h;
+#pragma unroll
+      for (int dblk = 0; dblk < 4; ++dblk)
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          *reinterpret_cast<f32x4*>(prow + 32 * dblk + 8 * w) =
+              f32x4{acc[dblk][4 * w], acc[dblk][4 * w + 1], acc[dblk][4 * w + 2], acc[dblk][4 * w + 3]};
+      __syncthreads();
+      constexpr int kPer = D / 4;  // threads per key
+      for (int it = tid; it < kKvBN * kPer; it += 64 * KW * QS) {
+        const int key = it / kPer, d = 4 * (it % kPer);
+        if (k0 + key >= a.Nk) break;
+        f32x4 sum = *reinterpret_cast<const f32x4*>(part + key * kPartPitch + d);
+#pragma unroll
+        for (int g = 1; g < QS; ++g)
+          sum += *reinterpret_cast<const f32x4*>(part + (g * kKvBN + key) * kPartPitch + d);
+        f32x4* p = reinterpret_cast<f32x4*>(out + (((int64_t)b * a.k_rows + k0 + key) * a.Hkv + hk) * D + d);
+        *p = *p + sum * scale;
       }
+    };
+    reduce(dk, a.dk, a.scale);
+    reduce(dv, a.dv, 1.f);
   }
 }
 
@@ -812,8 +884,24 @@ hipError_t launch_dkdv128(const Problem& p, const void* q, const void* k, const 
     a.ds_nqt = (p.Nq + kKvBM - 1) / kKvBM;
     a.ds_nkb = (p.Nk + kDsBlockKeys - 1) / kDsBlockKeys;
   }
-  a.n_tiles = (p.Nk + kKvBN - 1) / kKvBN;
-  hipLaunchKernelGGL(dkdv128_kernel, dim3(a.n_tiles * p.Hkv * p.B), dim3(256), 0, s, a);
+  const int64_t heads = (int64_t)p.Hkv * p.B;
+  // Few workgroups leave the chip idle, and with a diagonal the longest walk
+  // sets the time: four groups then split each walk (4,096 tokens, 32/8 heads,
+  // causal: 615 -> 361 us; 2,000 tokens, 16 heads 89 -> 63; 500 tokens, 32/8
+  // heads 88 -> 41; 8,192 tokens, 32/8 heads, 512 workgroups: 1350 -> 1210).
+  // They share tiles among two waves instead of four, so a grid that fills the
+  // chip evenly keeps one group (4,096 tokens, 16 heads, no diagonal, 512
+  // workgroups: 262 us against 372; causal 8,192 tokens, 16 heads, 1024: 555
+  // against 578).
+  const int64_t wgs = heads * ((p.Nk + 127) / 128);
+  const bool diagonal = p.causal && p.k_pos0 + p.Nk - 1 > p.q_pos0;
+  if (wgs <= (diagonal ? 512 : 128)) {
+    a.n_tiles = (p.Nk + 63) / 64;
+    hipLaunchKernelGGL((dkdv128_kernel<2, 4>), dim3(a.n_tiles * heads), dim3(512), 0, s, a);
+  } else {
+    a.n_tiles = (p.Nk + 127) / 128;
+    hipLaunchKernelGGL((dkdv128_kernel<4, 1>), dim3(a.n_tiles * heads), dim3(256), 0, s, a);
+  }
   return hipGetLastError();
 }
 
@@ -827,8 +915,18 @@ hipError_t launch_dqds128(const Problem& p, const void* k, const uint16_t* ds, i
   a.ds = const_cast<uint16_t*>(ds);
   a.ds_nqt = ds_nqt;
   a.ds_nkb = ds_nkb;
-  a.n_tiles = (p.Nq + kDsBM - 1) / kDsBM;
-  hipLaunchKernelGGL(dqds128_kernel, dim3(a.n_tiles * p.Hq * p.B), dim3(64 * kDsNW), 0, s, a);
+  const int64_t heads = (int64_t)p.Hq * p.B;
+  // Workgroups of four waves, two per CU, where 512-query ones would be at most
+  // one per CU (2,000 tokens, 16 heads: 73 -> 42 us; 2,048 tokens, 9 heads
+  // 92 -> 45; 4,096 x 4,096 tokens, 16 heads 185 -> 156); larger grids stream
+  // dS the faster the more waves share each K tile.
+  if (heads * ((p.Nq + 511) / 512) <= 256) {
+    a.n_tiles = (p.Nq + 127) / 128;
+    hipLaunchKernelGGL(dqds128_kernel<4>, dim3(a.n_tiles * heads), dim3(256), 0, s, a);
+  } else {
+    a.n_tiles = (p.Nq + 511) / 512;
+    hipLaunchKernelGGL(dqds128_kernel<16>, dim3(a.n_tiles * heads), dim3(1024), 0, s, a);
+  }
   return hipGetLastError();
 }
 
