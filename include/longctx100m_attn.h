@@ -91,6 +91,19 @@ typedef struct lc_attn_mask {
 int lc_attn_fwd_shard(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, const void* q,
                       const void* k, const void* v, float* o, float* m, float* l, void* stream);
 
+/* lc_attn_fwd_shard with a caller-owned workspace: a query shard whose
+ * workgroups alone would leave the chip idle (a prompt chunk of a few hundred
+ * tokens against many keys) has its keys split over more of them, and a second
+ * kernel merges the splits by log-sum-exp.  Applies to d = 128 on the bf16 MFMA
+ * path with up to 65,536 keys; lc_attn_fwd_shard_workspace_bytes returns the
+ * bytes it needs (at most 36 MB), 0 for shapes that do not split.  With a smaller or misaligned
+ * (16 bytes) workspace, or other shapes, this is lc_attn_fwd_shard.  Results
+ * agree up to fp32 summation order. */
+size_t lc_attn_fwd_shard_workspace_bytes(const lc_attn_shape_t* shape);
+int lc_attn_fwd_shard_ws(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, const void* q,
+                         const void* k, const void* v, float* o, float* m, float* l,
+                         void* workspace, size_t workspace_bytes, void* stream);
+
 /* Split-KV decode: the same outputs as lc_attn_fwd_shard for a query shard of
  * a few tokens against a long KV shard (a decode step over a KV cache).  For
  * bf16, head_dim 64 or 128 and q_tokens * heads_q / heads_kv <= 64 the key
@@ -209,6 +222,9 @@ typedef struct lc_ring_desc {
   int64_t q_position_start; /* -1 = None (defaults to rank * local_tokens) */
 } lc_ring_desc_t;
 
+/* Forward: the running fp32 output [B, n, Hq, D] (rounded up to 256 bytes),
+ * which is the least lc_ring_fwd_with_stats takes, plus the workspace of
+ * lc_attn_fwd_shard_ws for its hops. */
 size_t lc_ring_fwd_workspace_bytes(const lc_ring_desc_t* desc);
 size_t lc_ring_bwd_workspace_bytes(const lc_ring_desc_t* desc);
 /* Workspace for lc_ring_bwd that also holds the dS of the diagonal pair

@@ -122,11 +122,21 @@ bool pair_active(const lc::Problem& p) {
 // dV accumulate anyway.
 constexpr int64_t kStreamChunk = 65536;
 
+// Workspace with which the d = 128 bf16 forward splits the keys of a small
+// grid over the chip (0: it does not).
+size_t fwd_split_bytes(const lc::Problem& p) {
+  return p.D == 128 && lc::mfma_supported(p) && p.Nq > 0 && p.Nk <= kStreamChunk
+             ? lc::fwd128_split_bytes(p) : 0;
+}
+
 int fwd_shard(const lc::Problem& p, const void* q, const void* k, const void* v, float* o,
-              float* m, float* l, hipStream_t st) {
+              float* m, float* l, hipStream_t st, void* ws = nullptr, size_t ws_bytes = 0) {
   hipError_t e = hipSuccess;
   if (use_mfma(p, q, k, v, nullptr) && p.D == 128) {
-    if (p.Nk <= kStreamChunk) {
+    const size_t split = ws != nullptr && aligned16(ws) && aligned16(o) ? fwd_split_bytes(p) : 0;
+    if (split > 0 && ws_bytes >= split && lc::fwd128_splits(p) > 1) {
+      e = lc::launch_fwd128_split(p, q, k, v, o, m, l, ws, st);
+    } else if (p.Nk <= kStreamChunk) {
       e = lc::launch_fwd128(p, q, k, v, o, m, l, st, -1, p.accumulate);
     } else {
       const size_t row_bytes = (size_t)p.Hkv * p.D * 2;  // bf16 K/V row
@@ -348,12 +358,20 @@ const char* lc_last_error(void) { return g_last_error.c_str(); }
 
 int32_t lc_abi_version(void) { return 2; }
 
-int lc_attn_fwd_shard(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, const void* q,
-                      const void* k, const void* v, float* o, float* m, float* l, void* stream) {
+size_t lc_attn_fwd_shard_workspace_bytes(const lc_attn_shape_t* shape) {
+  if (check_shape(shape) != LC_OK) return 0;
+  return round_up(fwd_split_bytes(make_problem(shape, nullptr)));
+}
+
+int lc_attn_fwd_shard_ws(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, const void* q,
+                         const void* k, const void* v, float* o, float* m, float* l,
+                         void* workspace, size_t workspace_bytes, void* stream) {
   if (int rc = check_shape(shape)) return rc;
   if (!q || !k || !v || !o || !m || !l) return set_error(LC_ERR_INVALID, "null pointer argument");
   if (mask && mask->valid_length < -1)
     return set_error(LC_ERR_INVALID, "valid_length must be -1 (None) or non-negative");
+  if (workspace == nullptr && workspace_bytes != 0)
+    return set_error(LC_ERR_INVALID, "workspace is NULL but workspace_bytes is not 0");
   lc::Problem p = make_problem(shape, mask);
   p.accumulate = (shape->flags & LC_FLAG_ACCUMULATE) != 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -363,7 +381,12 @@ int lc_attn_fwd_shard(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, 
     hipError_t e = lc::launch_init_state(p.B, p.Nq, p.Hq, p.D, o, m, l, st);
     return e == hipSuccess ? LC_OK : hip_error(e, "lc_attn_fwd_shard init");
   }
-  return fwd_shard(p, q, k, v, o, m, l, st);
+  return fwd_shard(p, q, k, v, o, m, l, st, workspace, workspace_bytes);
+}
+
+int lc_attn_fwd_shard(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, const void* q,
+                      const void* k, const void* v, float* o, float* m, float* l, void* stream) {
+  return lc_attn_fwd_shard_ws(shape, mask, q, k, v, o, m, l, nullptr, 0, stream);
 }
 
 size_t lc_attn_decode_workspace_bytes(const lc_attn_shape_t* shape) {
@@ -556,7 +579,7 @@ int lc_attn_bwd_shard_ws(const lc_attn_shape_t* shape, const lc_attn_mask_t* mas
 
 size_t lc_ring_fwd_workspace_bytes(const lc_ring_desc_t* desc) {
   if (check_ring(desc) != LC_OK) return 0;
-  return fwd_ws_bytes(desc);
+  return fwd_ws_bytes(desc) + round_up(fwd_split_bytes(ring_problem(desc, 0, 0)));
 }
 
 size_t lc_ring_bwd_workspace_bytes(const lc_ring_desc_t* desc) {
@@ -611,7 +634,10 @@ int lc_ring_fwd_with_stats(const lc_ring_desc_t* d, const void* const* qs, const
     const int owner = owners[i];
     lc::Problem p = ring_problem(d, q_pos0, (int64_t)owner * n);
     p.accumulate = i > 0;
-    if (int rc = fwd_shard(p, qs[d->rank], ks[owner], vs[owner], o_run, m, l, st)) return rc;
+    if (int rc = fwd_shard(p, qs[d->rank], ks[owner], vs[owner], o_run, m, l, st,
+                           static_cast<char*>(workspace) + fwd_ws_bytes(d),
+                           workspace_bytes - fwd_ws_bytes(d)))
+      return rc;
   }
   LC_TRY_HIP(lc::launch_cast(o_run, out, (int64_t)n_o, d->dtype, st), "lc_ring_fwd_with_stats cast");
   return LC_OK;

@@ -44,6 +44,7 @@
 #include "kernels.h"
 #include "tile128.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace lc {
@@ -68,9 +69,13 @@ struct Fwd128Args {
   int causal;
   int accumulate;  // merge into the running (o, m, l) instead of writing them
   float sl2;       // scale * log2(e)
+  // Key splits: split s takes the keys from s * chunk and writes its (o, m, l)
+  // s * part_rows rows into them (the partials of merge_splits_kernel).
+  int splits, chunk;
+  int64_t part_rows;
 };
 
-template <int NW>
+template <int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void fwd128_kernel(Fwd128Args a) {
   constexpr int kWaves = NW;
   constexpr int BM = kWaves * kQW;  // queries per workgroup
@@ -83,7 +88,20 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void fwd128_kernel(Fwd128Args a) {
   const int kc = lane & 31;  // this lane's query within the wave
   const int hh = lane >> 5;  // which half of each 8-key group the lane holds
 
-  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  int L = xcd_remap(blockIdx.x, gridDim.x);
+  if constexpr (SPLIT) {  // this workgroup's keys and partial; the splits of a head lie apart
+    const int per = gridDim.x / a.splits;
+    const int sp = L / per;
+    L -= sp * per;
+    const int64_t k0 = (int64_t)sp * a.chunk, rows = (int64_t)a.Hkv * D;
+    a.k += k0 * rows;
+    a.v += k0 * rows;
+    a.Nk = (int)min((int64_t)a.chunk, a.Nk - k0);
+    a.k_pos0 += k0;
+    a.o += sp * a.part_rows * D;
+    a.m += sp * a.part_rows;
+    a.l += sp * a.part_rows;
+  }
   const int qt = a.n_qtiles - 1 - (L % a.n_qtiles);  // long query tiles first
   const int bh = L / a.n_qtiles;
   const int hq = bh % a.Hq;
@@ -331,12 +349,63 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void fwd128_kernel(Fwd128Args a) {
   }
 }
 
-}  // namespace
+// Merges the partials of each row, at most S (o normalised, its m and l) into the row's
+// (o, m, l): 32 threads per row, one 16-byte chunk each, every partial of the
+// chunk in flight.  accumulate: the result then merges into the running state.
+template <int S>
+__global__ __launch_bounds__(256) void merge_splits_kernel(int64_t rows, int splits, int N, int H,
+                                                           const float* po, const float* pm,
+                                                           const float* pl, float* o, float* m,
+                                                           float* l, int accumulate) {
+  const int64_t row = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);  // (b, n, h) of o
+  if (row >= rows) return;
+  const int d = 4 * (threadIdx.x & 31);
+  const int h = (int)(row % H);
+  const int64_t bn = row / H;
+  const int64_t si = (bn / N * H + h) * N + bn % N;
+  f32x4 x[S];
+  float ms[S], ls[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int64_t r = min(s, splits - 1) * rows;
+    x[s] = *reinterpret_cast<const f32x4*>(po + (r + row) * D + d);
+    ms[s] = s < splits ? pm[r + si] : -INFINITY;
+    ls[s] = pl[r + si];
+  }
+  float M = -INFINITY;
+#pragma unroll
+  for (int s = 0; s < S; ++s) M = fmaxf(M, ms[s]);
+  float L = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    if (ms[s] == -INFINITY) continue;  // the split saw no key
+    const float w = expf(ms[s] - M) * ls[s];
+    L += w;
+    acc += x[s] * w;
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  f32x4* dst = reinterpret_cast<f32x4*>(o + row * D + d);
+  if (accumulate) {
+    const MergeW w = merge_weights(m[si], l[si], M, L);
+    *dst = *dst * w.wa + acc * (inv * w.wb);
+    M = w.m;
+    L = w.l;
+  } else {
+    *dst = acc * inv;
+  }
+  if (d == 0) {  // the row's threads are in one wave: all have read the old statistics
+    m[si] = M;
+    l[si] = L;
+  }
+}
 
-hipError_t launch_fwd128(const Problem& p, const void* q, const void* k, const void* v, float* o,
-                         float* m, float* l, hipStream_t s, int64_t kv_rows, bool accumulate) {
-  if (p.D != D) return hipErrorInvalidValue;
-  Fwd128Args a;
+// No causal diagonal in the problem: every key precedes every query.
+bool no_diagonal(const Problem& p) { return !p.causal || p.k_pos0 + p.Nk - 1 <= p.q_pos0; }
+
+Fwd128Args make_args(const Problem& p, const void* q, const void* k, const void* v, float* o,
+                     float* m, float* l, int64_t kv_rows) {
+  Fwd128Args a{};
   a.q = static_cast<const uint16_t*>(q);
   a.k = static_cast<const uint16_t*>(k);
   a.v = static_cast<const uint16_t*>(v);
@@ -348,21 +417,79 @@ hipError_t launch_fwd128(const Problem& p, const void* q, const void* k, const v
   a.Hq = p.Hq;
   a.Hkv = p.Hkv;
   a.group = p.Hq / p.Hkv;
-  // No causal diagonal in this launch: every key precedes every query.
-  const bool full = !p.causal || p.k_pos0 + p.Nk - 1 <= p.q_pos0;
-  const int bm = (full ? 8 : 4) * kQW;
-  a.n_qtiles = (p.Nq + bm - 1) / bm;
+  a.n_qtiles = (p.Nq + (no_diagonal(p) ? 8 : 4) * kQW - 1) / ((no_diagonal(p) ? 8 : 4) * kQW);
   a.q_pos0 = p.q_pos0;
   a.k_pos0 = p.k_pos0;
   a.valid = p.valid;
   a.kv_bstride = (kv_rows < 0 ? p.Nk : kv_rows) * (int64_t)p.Hkv * D;
   a.causal = p.causal ? 1 : 0;
-  a.accumulate = accumulate ? 1 : 0;
   a.sl2 = p.scale * kLog2e;
-  if (full)
-    hipLaunchKernelGGL(fwd128_kernel<8>, dim3(a.n_qtiles * p.Hq * p.B), dim3(512), 0, s, a);
-  else
-    hipLaunchKernelGGL(fwd128_kernel<4>, dim3(a.n_qtiles * p.Hq * p.B), dim3(256), 0, s, a);
+  return a;
+}
+
+size_t split_bytes(const Problem& p, int S) {
+  const size_t rows = (size_t)p.B * p.Nq * p.Hq;
+  return S * rows * (D + 2) * sizeof(float);
+}
+
+}  // namespace
+
+// Splits of workgroups of `waves` waves, of at least 512 keys each: what the
+// chip holds at two waves per SIMD (512 queries, 32/8 heads over 32,512 keys:
+// 555 us in 128 workgroups of four waves, 281 in 512 and their merge; 17
+// queries over 20,017 keys 329 us and 35; 1,000 over 11,000 246 and 200), or,
+// where the keys do not suffice for most of that, one workgroup per CU (100
+// queries over 5,100 keys: 26.7 us in 256 against 32.6 in 288).
+static int splits_of(const Problem& p, int64_t waves) {
+  const int64_t wgs = (p.Nq + waves * kQW - 1) / (waves * kQW) * p.Hq * p.B;
+  int64_t s = std::min<int64_t>({256 * 8 / waves / wgs, p.Nk / kFwdSplitKeys, kFwdMaxSplits});
+  if (s * wgs > 256 && s * wgs < 400) s = 256 / wgs;
+  return (int)std::max<int64_t>(1, s);
+}
+
+int fwd128_splits(const Problem& p) { return splits_of(p, no_diagonal(p) ? 8 : 4); }
+
+size_t fwd128_split_bytes(const Problem& p) {
+  const int s = std::max(splits_of(p, 4), splits_of(p, 8));  // whatever the positions
+  return s > 1 ? split_bytes(p, s) : 0;
+}
+
+hipError_t launch_fwd128_split(const Problem& p, const void* q, const void* k, const void* v,
+                               float* o, float* m, float* l, void* ws, hipStream_t st) {
+  if (p.D != D) return hipErrorInvalidValue;
+  const int S = fwd128_splits(p);
+  const int64_t rows = (int64_t)p.B * p.Nq * p.Hq;
+  float* po = static_cast<float*>(ws);
+  float* pm = po + S * rows * D;
+  float* pl = pm + S * rows;
+  Fwd128Args a = make_args(p, q, k, v, po, pm, pl, -1);
+  a.splits = S;
+  a.chunk = ((p.Nk + S - 1) / S + BN - 1) / BN * BN;
+  a.splits = (p.Nk + a.chunk - 1) / a.chunk;  // no split without keys
+  a.part_rows = rows;
+  const dim3 grid((unsigned)(a.n_qtiles * p.Hq * p.B * a.splits));
+  if (no_diagonal(p)) hipLaunchKernelGGL((fwd128_kernel<8, true>), grid, dim3(512), 0, st, a);
+  else hipLaunchKernelGGL((fwd128_kernel<4, true>), grid, dim3(256), 0, st, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  auto merge = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, st, rows, a.splits,
+                       p.Nq, p.Hq, po, pm, pl, o, m, l, p.accumulate ? 1 : 0);
+  };
+  if (a.splits <= 4) merge(merge_splits_kernel<4>);
+  else if (a.splits <= 8) merge(merge_splits_kernel<8>);
+  else merge(merge_splits_kernel<kFwdMaxSplits>);
+  return hipGetLastError();
+}
+
+hipError_t launch_fwd128(const Problem& p, const void* q, const void* k, const void* v, float* o,
+                         float* m, float* l, hipStream_t s, int64_t kv_rows, bool accumulate) {
+  if (p.D != D) return hipErrorInvalidValue;
+  Fwd128Args a = make_args(p, q, k, v, o, m, l, kv_rows);
+  a.accumulate = accumulate ? 1 : 0;
+  const dim3 grid(a.n_qtiles * p.Hq * p.B);
+  if (no_diagonal(p)) hipLaunchKernelGGL((fwd128_kernel<8, false>), grid, dim3(512), 0, s, a);
+  else hipLaunchKernelGGL((fwd128_kernel<4, false>), grid, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

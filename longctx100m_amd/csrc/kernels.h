@@ -44,6 +44,15 @@ bool mfma_supported(const Problem& p);
 hipError_t launch_fwd128(const Problem& p, const void* q, const void* k, const void* v, float* o,
                          float* m, float* l, hipStream_t s, int64_t kv_rows = -1,
                          bool accumulate = false);
+// Small grids: the keys in up to kFwdMaxSplits splits of at least
+// kFwdSplitKeys, as many as the chip holds workgroups for, whose partials lie in a workspace
+// of fwd128_split_bytes (0: one split) and are merged by a second kernel.
+constexpr int kFwdMaxSplits = 16;
+constexpr int64_t kFwdSplitKeys = 512;
+int fwd128_splits(const Problem& p);
+size_t fwd128_split_bytes(const Problem& p);
+hipError_t launch_fwd128_split(const Problem& p, const void* q, const void* k, const void* v,
+                               float* o, float* m, float* l, void* ws, hipStream_t s);
 // The backward can run on a sub-shard too (results accumulate into dq, dk,
 // dv anyway): dQ on a key sub-shard (k, v at its first key, k_rows = keys of
 // the whole shard), dK/dV on a query sub-shard (q, dout, lse2, delta at its

@@ -115,8 +115,15 @@ def fwd_shard(q, k, v, *, q_pos0: int, k_pos0: int, causal: bool = True,
     m = torch.empty((b, hq, nq), dtype=torch.float32, device=q.device) if m is None else m
     l = torch.empty((b, hq, nq), dtype=torch.float32, device=q.device) if l is None else l
     mk = _lib.Mask(q_pos0, k_pos0, _opt(valid_length), int(causal), 0)
-    _lib.check(_lib.load().lc_attn_fwd_shard(s, mk, q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                             o.data_ptr(), m.data_ptr(), l.data_ptr(), _stream()))
+    lib = _lib.load()
+    ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), m.data_ptr(), l.data_ptr())
+    # scratch with which a small grid's keys are split over the chip
+    need = lib.lc_attn_fwd_shard_workspace_bytes(s) if d == 128 else 0
+    if need:
+        ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+        _lib.check(lib.lc_attn_fwd_shard_ws(s, mk, *ptrs, ws.data_ptr(), need, _stream()))
+    else:
+        _lib.check(lib.lc_attn_fwd_shard(s, mk, *ptrs, _stream()))
     return o, m, l
 
 
