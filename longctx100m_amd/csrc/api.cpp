@@ -129,15 +129,17 @@ size_t fwd_split_bytes(const lc::Problem& p) {
              ? lc::fwd128_split_bytes(p) : 0;
 }
 
+// out: o goes there as bf16 instead (shards of at most kStreamChunk keys).
 int fwd_shard(const lc::Problem& p, const void* q, const void* k, const void* v, float* o,
-              float* m, float* l, hipStream_t st, void* ws = nullptr, size_t ws_bytes = 0) {
+              float* m, float* l, hipStream_t st, void* ws = nullptr, size_t ws_bytes = 0,
+              uint16_t* out = nullptr) {
   hipError_t e = hipSuccess;
   if (use_mfma(p, q, k, v, nullptr) && p.D == 128) {
     const size_t split = ws != nullptr && aligned16(ws) && aligned16(o) ? fwd_split_bytes(p) : 0;
     if (split > 0 && ws_bytes >= split && lc::fwd128_splits(p) > 1) {
-      e = lc::launch_fwd128_split(p, q, k, v, o, m, l, ws, st);
+      e = lc::launch_fwd128_split(p, q, k, v, o, m, l, ws, st, out);
     } else if (p.Nk <= kStreamChunk) {
-      e = lc::launch_fwd128(p, q, k, v, o, m, l, st, -1, p.accumulate);
+      e = lc::launch_fwd128(p, q, k, v, o, m, l, st, -1, p.accumulate, out);
     } else {
       const size_t row_bytes = (size_t)p.Hkv * p.D * 2;  // bf16 K/V row
       bool first = true;
@@ -153,27 +155,29 @@ int fwd_shard(const lc::Problem& p, const void* q, const void* k, const void* v,
       }
     }
   } else if (use_mfma(p, q, k, v, nullptr)) {
-    e = lc::launch_fwd64(p, q, k, v, o, m, l, st);
+    e = lc::launch_fwd64(p, q, k, v, o, m, l, st, out);
   } else {
-    e = lc::launch_fwd_generic(p, q, k, v, o, m, l, st);
+    e = lc::launch_fwd_generic(p, q, k, v, o, m, l, st, out);
   }
   if (e != hipSuccess) return hip_error(e, "lc_attn_fwd_shard launch");
   return LC_OK;
 }
 
+// to applies to the one of dq and (dk, dv) that is set, on shards of at most
+// kStreamChunk tokens.
 int bwd_shard(const lc::Problem& p, const void* q, const void* k, const void* v, const void* dout,
               const float* lse2, const float* delta, float* dq, float* dk, float* dv,
-              hipStream_t st) {
+              hipStream_t st, const lc::Sink& to = {}) {
   const bool mf = use_mfma(p, q, k, v, dout);
   const bool d128 = p.D == 128;
   if (dq != nullptr) {
     hipError_t e = hipSuccess;
     if (!mf) {
-      e = lc::launch_bwd_dq_generic(p, q, k, v, dout, lse2, delta, dq, st);
+      e = lc::launch_bwd_dq_generic(p, q, k, v, dout, lse2, delta, dq, st, to);
     } else if (!d128) {
-      e = lc::launch_dq64(p, q, k, v, dout, lse2, delta, dq, st);
+      e = lc::launch_dq64(p, q, k, v, dout, lse2, delta, dq, st, to);
     } else if (p.Nk <= kStreamChunk) {
-      e = lc::launch_dq128(p, q, k, v, dout, lse2, delta, dq, st);
+      e = lc::launch_dq128(p, q, k, v, dout, lse2, delta, dq, st, -1, to);
     } else {  // key sub-shards
       const size_t row_bytes = (size_t)p.Hkv * p.D * 2;
       for (int64_t c0 = 0; c0 < p.Nk && e == hipSuccess; c0 += kStreamChunk) {
@@ -191,11 +195,11 @@ int bwd_shard(const lc::Problem& p, const void* q, const void* k, const void* v,
   if (dk != nullptr) {
     hipError_t e = hipSuccess;
     if (!mf) {
-      e = lc::launch_bwd_dkdv_generic(p, q, k, v, dout, lse2, delta, dk, dv, st);
+      e = lc::launch_bwd_dkdv_generic(p, q, k, v, dout, lse2, delta, dk, dv, st, to);
     } else if (!d128) {
-      e = lc::launch_dkdv64(p, q, k, v, dout, lse2, delta, dk, dv, st);
+      e = lc::launch_dkdv64(p, q, k, v, dout, lse2, delta, dk, dv, st, to);
     } else if (p.Nq <= kStreamChunk) {
-      e = lc::launch_dkdv128(p, q, k, v, dout, lse2, delta, dk, dv, st);
+      e = lc::launch_dkdv128(p, q, k, v, dout, lse2, delta, dk, dv, st, -1, nullptr, to);
     } else {  // query sub-shards
       const size_t row_bytes = (size_t)p.Hq * p.D * 2;
       for (int64_t c0 = 0; c0 < p.Nq && e == hipSuccess; c0 += kStreamChunk) {
@@ -247,9 +251,11 @@ bool ds_path(const lc::Problem& p, const void* q, const void* k, const void* v, 
   return p.D == 128 && use_mfma(p, q, k, v, dout);
 }
 
+// to_kv, to_q: only when one chunk and one key sub-shard are the whole pair.
 int bwd_shard_ds(const lc::Problem& p, int64_t chunk, const void* q, const void* k, const void* v,
                  const void* dout, const float* lse2, const float* delta, float* dq, float* dk,
-                 float* dv, uint16_t* ds, hipStream_t st) {
+                 float* dv, uint16_t* ds, hipStream_t st, const lc::Sink& to_kv = {},
+                 const lc::Sink& to_q = {}) {
   const size_t qrow_bytes = (size_t)p.Hq * p.D * 2;  // bf16 Q / dO row
   const size_t krow_bytes = (size_t)p.Hkv * p.D * 2;
   const int nkb = (p.Nk + 31) / 32;
@@ -260,7 +266,7 @@ int bwd_shard_ds(const lc::Problem& p, int64_t chunk, const void* q, const void*
     if (!pair_active(pc)) continue;
     hipError_t e = lc::launch_dkdv128(pc, static_cast<const char*>(q) + c0 * qrow_bytes, k, v,
                                       static_cast<const char*>(dout) + c0 * qrow_bytes, lse2 + c0,
-                                      delta + c0, dk, dv, st, p.Nq, ds);
+                                      delta + c0, dk, dv, st, p.Nq, ds, to_kv);
     if (e != hipSuccess) return hip_error(e, "lc_attn_bwd_shard_ws dk/dv launch");
     const int nqt = (pc.Nq + 31) / 32;
     float* dqc = dq + c0 * p.Hq * p.D;
@@ -270,7 +276,7 @@ int bwd_shard_ds(const lc::Problem& p, int64_t chunk, const void* q, const void*
       pk.k_pos0 = p.k_pos0 + k0;
       if (!pair_active(pk)) continue;
       e = lc::launch_dqds128(pk, static_cast<const char*>(k) + k0 * krow_bytes,
-                             ds + (k0 / 32) * 1024, nqt, nkb, dqc, st, p.Nk, p.Nq);
+                             ds + (k0 / 32) * 1024, nqt, nkb, dqc, st, p.Nk, p.Nq, to_q);
     }
     if (e != hipSuccess) return hip_error(e, "lc_attn_bwd_shard_ws dq launch");
   }
@@ -336,6 +342,12 @@ int check_ptrs(const void* const* arr, int world, const char* what) {
   for (int i = 0; i < world; ++i)
     if (arr[i] == nullptr) return set_error(LC_ERR_INVALID, "null %s[%d]", what, i);
   return LC_OK;
+}
+
+// Whether [a, a + na) and [b, b + nb) have no byte in common.
+bool apart(const void* a, size_t na, const void* b, size_t nb) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x + na <= y || y + nb <= x;
 }
 
 // Device buffer owned for the duration of a host-pointer call.
@@ -611,7 +623,17 @@ int lc_ring_fwd_with_stats(const lc_ring_desc_t* d, const void* const* qs, const
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int n = d->local_tokens;
   const size_t n_o = (size_t)d->batch * n * d->heads_q * d->head_dim;
-  float* o_run = static_cast<float*>(workspace);
+  // fp32 results are run in place; bf16 ones are written by the last hop (the
+  // running fp32 output, one more read of it and a cast kernel are then only
+  // needed between hops).  An output that lies over an input is written last,
+  // by the cast.
+  const bool f32 = d->dtype == LC_DTYPE_F32;
+  const size_t q_bytes = n_o * dtype_size(d->dtype), kv_bytes = q_bytes / d->heads_q * d->heads_kv;
+  bool clear = aligned16(out) && apart(out, q_bytes, qs[d->rank], q_bytes);
+  for (int i = 0; i < d->world; ++i)
+    clear = clear && apart(out, q_bytes, ks[i], kv_bytes) && apart(out, q_bytes, vs[i], kv_bytes);
+  float* o_run = f32 && clear ? static_cast<float*>(out) : static_cast<float*>(workspace);
+  const bool direct = !f32 && clear && n <= kStreamChunk;
   const int64_t q_pos0 = d->q_position_start >= 0 ? d->q_position_start : (int64_t)d->rank * n;
 
   // Hops with at least one unmasked pair; the others leave the reference's
@@ -624,7 +646,8 @@ int lc_ring_fwd_with_stats(const lc_ring_desc_t* d, const void* const* qs, const
   if (owners.empty()) {
     LC_TRY_HIP(lc::launch_init_state(d->batch, n, d->heads_q, d->head_dim, o_run, m, l, st),
                "lc_ring_fwd_with_stats init");
-    LC_TRY_HIP(lc::launch_cast(o_run, out, (int64_t)n_o, d->dtype, st), "lc_ring_fwd_with_stats cast");
+    if (o_run != out)
+      LC_TRY_HIP(lc::launch_cast(o_run, out, (int64_t)n_o, d->dtype, st), "lc_ring_fwd_with_stats cast");
     return LC_OK;
   }
   // The first hop writes (o_run, m, l); every later hop LSE-merges its result
@@ -636,9 +659,11 @@ int lc_ring_fwd_with_stats(const lc_ring_desc_t* d, const void* const* qs, const
     p.accumulate = i > 0;
     if (int rc = fwd_shard(p, qs[d->rank], ks[owner], vs[owner], o_run, m, l, st,
                            static_cast<char*>(workspace) + fwd_ws_bytes(d),
-                           workspace_bytes - fwd_ws_bytes(d)))
+                           workspace_bytes - fwd_ws_bytes(d),
+                           direct && i + 1 == owners.size() ? static_cast<uint16_t*>(out) : nullptr))
       return rc;
   }
+  if (direct || o_run == out) return LC_OK;
   LC_TRY_HIP(lc::launch_cast(o_run, out, (int64_t)n_o, d->dtype, st), "lc_ring_fwd_with_stats cast");
   return LC_OK;
 }
@@ -676,10 +701,6 @@ int lc_ring_bwd(const lc_ring_desc_t* d, const void* const* qs, const void* cons
   w += round_up(n_s * 4);
   float* lse2 = reinterpret_cast<float*>(w);
 
-  LC_TRY_HIP(lc::launch_fill_zero(dq_acc, (int64_t)n_q, st), "lc_ring_bwd zero");
-  LC_TRY_HIP(lc::launch_fill_zero(dk_acc, (int64_t)n_k, st), "lc_ring_bwd zero");
-  LC_TRY_HIP(lc::launch_fill_zero(dv_acc, (int64_t)n_k, st), "lc_ring_bwd zero");
-
   // The diagonal pair (this rank's queries against this rank's keys) is hop 0
   // of both passes: pass 1 takes its dK/dV, pass 2 its dQ, with the same
   // positions when q_position_start is the default.  Given workspace beyond
@@ -695,51 +716,106 @@ int lc_ring_bwd(const lc_ring_desc_t* d, const void* const* qs, const void* cons
     ds = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + bwd_ws_bytes(d));
     ds_chunk = ds_chunk_rows(pd, workspace_bytes - bwd_ws_bytes(d));
   }
+
+  // The hops that contribute to dk and dv (pass 1) and to dq (pass 2), in order.
+  std::vector<int> kv_hops, q_hops;
+  for (int hop = 0; hop < d->world; ++hop) {
+    const int o = ((r - hop) % d->world + d->world) % d->world;
+    if (o == r && ds_chunk > 0) continue;  // the shared diagonal pair, before both
+    if (pair_active(ring_problem(d, (int64_t)o * n, (int64_t)r * n))) kv_hops.push_back(o);
+    if (pair_active(ring_problem(d, q_pos0, (int64_t)o * n))) q_hops.push_back(o);
+  }
+  // With one launch per hop the first contribution initialises the accumulator
+  // and the last one writes the result in the output's dtype (fp32 results
+  // accumulate in place), so neither is zeroed, read back nor cast in passes
+  // of its own.
+  const bool f32 = d->dtype == LC_DTYPE_F32;
+  bool single = n <= kStreamChunk && (ds_chunk == 0 || ds_chunk >= n) && aligned16(dq) &&
+                aligned16(dk) && aligned16(dv);
+  // ... unless a result lies over an input that a later launch reads.
+  const size_t q_bytes = n_q * dtype_size(d->dtype), kv_bytes = n_k * dtype_size(d->dtype);
+  auto clear_of = [&](const void* res, size_t bytes) {
+    for (int i = 0; i < d->world; ++i)
+      if (!apart(res, bytes, qs[i], q_bytes) || !apart(res, bytes, ks[i], kv_bytes) ||
+          !apart(res, bytes, vs[i], kv_bytes) || !apart(res, bytes, outs[i], q_bytes) ||
+          !apart(res, bytes, grad_outs[i], q_bytes) || !apart(res, bytes, ms[i], n_s * 4) ||
+          !apart(res, bytes, ls[i], n_s * 4))
+        return false;
+    return true;
+  };
+  single = single && clear_of(dq, q_bytes) && clear_of(dk, kv_bytes) && clear_of(dv, kv_bytes);
+  const bool direct_q = single && (ds_chunk > 0 || !q_hops.empty());
+  const bool direct_kv = single && (ds_chunk > 0 || !kv_hops.empty());
+  if (direct_q && f32) dq_acc = static_cast<float*>(dq);
+  if (direct_kv && f32) {
+    dk_acc = static_cast<float*>(dk);
+    dv_acc = static_cast<float*>(dv);
+  }
+  if (!direct_q)
+    LC_TRY_HIP(lc::launch_fill_zero(dq_acc, (int64_t)n_q, st), "lc_ring_bwd zero");
+  if (!direct_kv) {
+    LC_TRY_HIP(lc::launch_fill_zero(dk_acc, (int64_t)n_k, st), "lc_ring_bwd zero");
+    LC_TRY_HIP(lc::launch_fill_zero(dv_acc, (int64_t)n_k, st), "lc_ring_bwd zero");
+  }
+  auto sink_q = [&](bool first, bool last) {
+    lc::Sink t;
+    t.init = direct_q && first;
+    if (direct_q && last && !f32) t.out = static_cast<uint16_t*>(dq);
+    return t;
+  };
+  auto sink_kv = [&](bool first, bool last) {
+    lc::Sink t;
+    t.init = direct_kv && first;
+    if (direct_kv && last && !f32) {
+      t.out = static_cast<uint16_t*>(dk);
+      t.out2 = static_cast<uint16_t*>(dv);
+    }
+    return t;
+  };
+  int stats_of = -1;  // owner whose statistics delta and lse2 hold
+  auto preprocess = [&](int o) {
+    if (stats_of == o) return (int)LC_OK;
+    stats_of = o;
+    hipError_t e = lc::launch_bwd_preprocess(d->batch, n, d->heads_q, d->head_dim, d->dtype,
+                                             outs[o], grad_outs[o], ms[o], ls[o], delta, lse2, st);
+    return e == hipSuccess ? (int)LC_OK : hip_error(e, "lc_ring_bwd preprocess");
+  };
   if (ds_chunk > 0) {
-    LC_TRY_HIP(lc::launch_bwd_preprocess(d->batch, n, d->heads_q, d->head_dim, d->dtype, outs[r],
-                                         grad_outs[r], ms[r], ls[r], delta, lse2, st),
-               "lc_ring_bwd preprocess");
+    if (int rc = preprocess(r)) return rc;
     if (int rc = bwd_shard_ds(pd, ds_chunk, qs[r], ks[r], vs[r], grad_outs[r], lse2, delta,
-                              dq_acc, dk_acc, dv_acc, ds, st))
+                              dq_acc, dk_acc, dv_acc, ds, st, sink_kv(true, kv_hops.empty()),
+                              sink_q(true, q_hops.empty())))
       return rc;
   }
 
   // Pass 1 (rs:367-416): local KV fixed, query owners rank, rank-1, ...;
   // query positions owner*n + i.
-  bool pass1_stats = false;  // delta / lse2 hold another owner's statistics
-  for (int hop = 0; hop < d->world; ++hop) {
-    const int qo = ((r - hop) % d->world + d->world) % d->world;
-    if (qo == r && ds_chunk > 0) continue;  // done above
-    const lc::Problem p = ring_problem(d, (int64_t)qo * n, (int64_t)r * n);
-    if (!pair_active(p)) continue;
-    pass1_stats = true;
-    LC_TRY_HIP(lc::launch_bwd_preprocess(d->batch, n, d->heads_q, d->head_dim, d->dtype, outs[qo],
-                                         grad_outs[qo], ms[qo], ls[qo], delta, lse2, st),
-               "lc_ring_bwd preprocess");
-    if (int rc = bwd_shard(p, qs[qo], ks[r], vs[r], grad_outs[qo], lse2, delta, nullptr, dk_acc,
-                           dv_acc, st))
+  for (size_t i = 0; i < kv_hops.size(); ++i) {
+    const int qo = kv_hops[i];
+    if (int rc = preprocess(qo)) return rc;
+    if (int rc = bwd_shard(ring_problem(d, (int64_t)qo * n, (int64_t)r * n), qs[qo], ks[r], vs[r],
+                           grad_outs[qo], lse2, delta, nullptr, dk_acc, dv_acc, st,
+                           sink_kv(i == 0 && ds_chunk == 0, i + 1 == kv_hops.size())))
       return rc;
   }
 
   // Pass 2 (rs:418-460): local Q fixed with positions q_position_start
   // (default rank*n) + i, KV owners rank, rank-1, ...
-  if (ds_chunk == 0 || pass1_stats)
-    LC_TRY_HIP(lc::launch_bwd_preprocess(d->batch, n, d->heads_q, d->head_dim, d->dtype, outs[r],
-                                         grad_outs[r], ms[r], ls[r], delta, lse2, st),
-               "lc_ring_bwd preprocess");
-  for (int hop = 0; hop < d->world; ++hop) {
-    const int owner = ((r - hop) % d->world + d->world) % d->world;
-    if (owner == r && ds_chunk > 0) continue;  // done above
-    const lc::Problem p = ring_problem(d, q_pos0, (int64_t)owner * n);
-    if (!pair_active(p)) continue;
-    if (int rc = bwd_shard(p, qs[r], ks[owner], vs[owner], grad_outs[r], lse2, delta, dq_acc,
-                           nullptr, nullptr, st))
+  for (size_t i = 0; i < q_hops.size(); ++i) {
+    const int owner = q_hops[i];
+    if (int rc = preprocess(r)) return rc;
+    if (int rc = bwd_shard(ring_problem(d, q_pos0, (int64_t)owner * n), qs[r], ks[owner],
+                           vs[owner], grad_outs[r], lse2, delta, dq_acc, nullptr, nullptr, st,
+                           sink_q(i == 0 && ds_chunk == 0, i + 1 == q_hops.size())))
       return rc;
   }
 
-  LC_TRY_HIP(lc::launch_cast(dq_acc, dq, (int64_t)n_q, d->dtype, st), "lc_ring_bwd cast");
-  LC_TRY_HIP(lc::launch_cast(dk_acc, dk, (int64_t)n_k, d->dtype, st), "lc_ring_bwd cast");
-  LC_TRY_HIP(lc::launch_cast(dv_acc, dv, (int64_t)n_k, d->dtype, st), "lc_ring_bwd cast");
+  if (!direct_q)
+    LC_TRY_HIP(lc::launch_cast(dq_acc, dq, (int64_t)n_q, d->dtype, st), "lc_ring_bwd cast");
+  if (!direct_kv) {
+    LC_TRY_HIP(lc::launch_cast(dk_acc, dk, (int64_t)n_k, d->dtype, st), "lc_ring_bwd cast");
+    LC_TRY_HIP(lc::launch_cast(dv_acc, dv, (int64_t)n_k, d->dtype, st), "lc_ring_bwd cast");
+  }
   return LC_OK;
 }
 

@@ -75,6 +75,8 @@ struct Args64 {
   int accumulate;  // forward: merge into the running (o, m, l) instead of writing them
   float sl2;       // scale * log2(e)
   float scale;
+  int init;                      // backward: replace the accumulators' contents
+  uint16_t *out, *dk16, *dv16;   // set: o (dQ), dK, dV go here as bf16 instead
 };
 
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
@@ -347,17 +349,18 @@ __global__ __launch_bounds__(64 * W, 2) void fwd64_kernel(Args64 a) {
       const float ltrue = lt > 0.f ? lt * fast_exp2(rtop[p0][r] - top) : 0.f;
       const float mnat = top == -INFINITY ? -INFINITY : top * kLn2;
       const int64_t si = ((int64_t)b * a.Hq + h) * a.Nq + row;
-      f32x4* dst = reinterpret_cast<f32x4*>(a.o + (((int64_t)b * a.Nq + row) * a.Hq + h) * D + d);
+      const int64_t oi = (((int64_t)b * a.Nq + row) * a.Hq + h) * D + d;
+      uint16_t* out = a.out != nullptr ? a.out + oi : nullptr;
       if (a.accumulate) {
         const MergeW w = merge_weights(a.m[si], a.l[si], mnat, ltrue);
-        *dst = *dst * w.wa + acc * (w.wb * inv);
+        store4(a.o + oi, out, *reinterpret_cast<const f32x4*>(a.o + oi) * w.wa + acc * (w.wb * inv));
         // every thread of the row has read the old statistics: they are in one wave
         if (d == 0) {
           a.m[si] = w.m;
           a.l[si] = w.l;
         }
       } else {
-        *dst = acc * inv;
+        store4(a.o + oi, out, acc * inv);
         if (d == 0) {
           a.m[si] = mnat;
           a.l[si] = ltrue;
@@ -390,7 +393,8 @@ __global__ __launch_bounds__(64 * W, 2) void dq64_kernel(Args64 a) {
   const uint16_t* kb = a.k + (int64_t)b * a.Nk * ks + (int64_t)hk * D;
   const uint16_t* vb = a.v + (int64_t)b * a.Nk * ks + (int64_t)hk * D;
 
-  if (visible_keys(a, min(qt * rows_wg + rows_wg, a.Nq) - 1) == 0) return;  // no contribution
+  if (visible_keys(a, min(qt * rows_wg + rows_wg, a.Nq) - 1) == 0 && !a.init && a.out == nullptr)
+    return;  // no contribution
   const int q0 = qt * rows_wg + qsub * kRows * NQ;
   const int kend = q0 < a.Nq ? visible_keys(a, min(q0 + kRows * NQ, a.Nq) - 1) : 0;
   const int kall = q0 < a.Nq ? visible_keys(a, q0) : 0;
@@ -478,8 +482,8 @@ __global__ __launch_bounds__(64 * W, 2) void dq64_kernel(Args64 a) {
       const int row = q0 + kRows * n + r;
       if (row >= a.Nq) break;
       const int d = 4 * (lane & 15);
-      f32x4* dst = reinterpret_cast<f32x4*>(a.dq + (((int64_t)b * a.Nq + row) * a.Hq + h) * D + d);
-      *dst = *dst + sum_parts<W>(smem, qsub * a.split, a.split, r * kPitch + d);
+      grad4(a.dq, a.out, a.init, (((int64_t)b * a.Nq + row) * a.Hq + h) * D + d,
+            sum_parts<W>(smem, qsub * a.split, a.split, r * kPitch + d));
     }
   }
 }
@@ -514,7 +518,8 @@ __global__ __launch_bounds__(64 * W, 2) void dkdv64_kernel(Args64 a) {
     const int64_t first = a.k_pos0 + key - a.q_pos0;
     return first <= 0 ? 0 : (first >= a.Nq ? a.Nq : (int)first);
   };
-  if (first_query(kt * keys_wg) >= a.Nq) return;  // no visible pair: no contribution
+  if (first_query(kt * keys_wg) >= a.Nq && !a.init && a.dk16 == nullptr)
+    return;  // no visible pair: no contribution
   const int k0 = kt * keys_wg + ksub * kRows;
   const int qstart = first_query(k0) / kRows * kRows;
   const int qall = first_query(k0 + kRows - 1);  // queries from here on see all the wave's keys
@@ -625,10 +630,9 @@ __global__ __launch_bounds__(64 * W, 2) void dkdv64_kernel(Args64 a) {
     if (k0 + r >= a.Nk) break;
     const int d = 4 * (lane & 15);
     const int64_t off = (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D + d;
-    f32x4* pk = reinterpret_cast<f32x4*>(a.dk + off);
-    f32x4* pv = reinterpret_cast<f32x4*>(a.dv + off);
-    *pk = *pk + sum_parts<W>(smem, ksub * a.split, a.split, r * kPitch + d);
-    *pv = *pv + sum_parts<W>(smem, ksub * a.split, a.split, kPart + r * kPitch + d);
+    grad4(a.dk, a.dk16, a.init, off, sum_parts<W>(smem, ksub * a.split, a.split, r * kPitch + d));
+    grad4(a.dv, a.dv16, a.init, off,
+          sum_parts<W>(smem, ksub * a.split, a.split, kPart + r * kPitch + d));
   }
 }
 
@@ -683,9 +687,10 @@ bool mfma_supported(const Problem& p) {
 }
 
 hipError_t launch_fwd64(const Problem& p, const void* q, const void* k, const void* v, float* o,
-                        float* m, float* l, hipStream_t s) {
+                        float* m, float* l, hipStream_t s, uint16_t* out) {
   if (p.D != D) return hipErrorInvalidValue;
   Args64 a = make_args(p, q, k, v, nullptr);
+  a.out = out;
   a.o = o;
   a.m = m;
   a.l = l;
@@ -704,9 +709,11 @@ hipError_t launch_fwd64(const Problem& p, const void* q, const void* k, const vo
 
 hipError_t launch_dq64(const Problem& p, const void* q, const void* k, const void* v,
                        const void* dout, const float* lse2, const float* delta, float* dq,
-                       hipStream_t s) {
+                       hipStream_t s, const Sink& to) {
   if (p.D != D) return hipErrorInvalidValue;
   Args64 a = make_args(p, q, k, v, dout);
+  a.init = to.init;
+  a.out = to.out;
   a.lse2 = lse2;
   a.delta = delta;
   a.dq = dq;
@@ -725,9 +732,12 @@ hipError_t launch_dq64(const Problem& p, const void* q, const void* k, const voi
 
 hipError_t launch_dkdv64(const Problem& p, const void* q, const void* k, const void* v,
                          const void* dout, const float* lse2, const float* delta, float* dk,
-                         float* dv, hipStream_t s) {
+                         float* dv, hipStream_t s, const Sink& to) {
   if (p.D != D) return hipErrorInvalidValue;
   Args64 a = make_args(p, q, k, v, dout);
+  a.init = to.init;
+  a.dk16 = to.out;
+  a.dv16 = to.out2;
   a.lse2 = lse2;
   a.delta = delta;
   a.dk = dk;

@@ -60,6 +60,8 @@ struct Bwd128Args {
   // them): ds_nqt query tiles x ds_nkb key blocks per (batch, query head).
   uint16_t* ds;
   int ds_nqt, ds_nkb;
+  int init;                        // replace the accumulators' contents
+  uint16_t *dq16, *dk16, *dv16;    // set: the gradients go here as bf16 instead
 };
 
 // dS exchange layout.  dS (bf16, unscaled) of query tile qt (32 queries) and
@@ -130,13 +132,15 @@ __global__ __launch_bounds__(256, 2) void dq128_kernel(Bwd128Args a) {
   if (a.causal) kend = min(kend, a.q_pos0 + q_end - a.k_pos0);
   kend = min(kend, a.valid - a.k_pos0);
   const int ntiles = kend > 0 ? (int)((kend + kDqBN - 1) / kDqBN) : 0;
-  if (ntiles == 0) return;  // nothing visible: dQ gets no contribution
+  if (ntiles == 0 && !a.init && a.dq16 == nullptr) return;  // nothing visible: no contribution
 
   const uint32_t smem_lds = t128::lds_addr(smem);
   t128::RowLoader<kDqBN, 4> ld;
   ld.init(ks, wave, lane);
-  ld.load(kbase, ks, 0, a.Nk, smem_lds, wave, lane);
-  ld.load(vbase, ks, 0, a.Nk, smem_lds + kDqTile, wave, lane);
+  if (ntiles > 0) {
+    ld.load(kbase, ks, 0, a.Nk, smem_lds, wave, lane);
+    ld.load(vbase, ks, 0, a.Nk, smem_lds + kDqTile, wave, lane);
+  }
 
   // Q^T, dO^T as B operands: lane holds query qw0 + kc, dims 16t + 8hh .. +7.
   bf16x8 qreg[D / 16], doreg[D / 16];
@@ -272,14 +276,13 @@ __global__ __launch_bounds__(256, 2) void dq128_kernel(Bwd128Args a) {
   // dQ^T element v of lane l: query qw0 + kc, dim 32*dblk + 8(v/4) + 4hh + v%4.
   const int row = qw0 + kc;
   if (row < a.Nq) {
-    float* dst = a.dq + (((int64_t)b * a.q_rows + row) * a.Hq + h) * D;
+    const int64_t qi = (((int64_t)b * a.q_rows + row) * a.Hq + h) * D;
 #pragma unroll
     for (int d = 0; d < 4; ++d)
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        f32x4* p = reinterpret_cast<f32x4*>(dst + 32 * d + 8 * w + 4 * hh);
         const f32x4 v4 = {acc[d][4 * w], acc[d][4 * w + 1], acc[d][4 * w + 2], acc[d][4 * w + 3]};
-        *p = *p + v4 * a.scale;
+        grad4(a.dq, a.dq16, a.init, qi + 32 * d + 8 * w + 4 * hh, v4 * a.scale);
       }
   }
 }
@@ -343,7 +346,7 @@ __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
   if (a.causal) kend = min(kend, a.q_pos0 + q_end - a.k_pos0);
   kend = min(kend, a.valid - a.k_pos0);
   const int ntiles = kend > 0 ? (int)((kend + kDqBN - 1) / kDqBN) : 0;
-  if (ntiles == 0) return;
+  if (ntiles == 0 && !a.init && a.dq16 == nullptr) return;
   int nt_w = 0;
   if (qw0 < a.Nq) {
     int64_t kw = kend;
@@ -374,7 +377,7 @@ __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
       t128::dma_b128_nt(src + si * (kDsBlockElems / 2), 16u * lane, dst + i * 1024);
     }
   };
-  ld.load(kbase, ks, 0, a.Nk, kbuf_lds, wave, lane);
+  if (ntiles > 0) ld.load(kbase, ks, 0, a.Nk, kbuf_lds, wave, lane);
   load_ds(0);
   if constexpr (kDsStages == 3) load_ds(1);
 
@@ -432,15 +435,14 @@ __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
 
   // dQ^T element v of lane l: query qw0 + ds_query(l % 32), dim 32 dblk + 8(v/4) + 4hh + v%4.
   const int row = qw0 + ds_query(kc);
-  if (nt_w > 0 && row < a.Nq) {
-    float* dst = a.dq + (((int64_t)b * a.q_rows + row) * a.Hq + h) * D;
+  if ((nt_w > 0 || a.init || a.dq16 != nullptr) && row < a.Nq) {
+    const int64_t qi = (((int64_t)b * a.q_rows + row) * a.Hq + h) * D;
 #pragma unroll
     for (int d = 0; d < 4; ++d)
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        f32x4* p = reinterpret_cast<f32x4*>(dst + 32 * d + 8 * w + 4 * hh);
         const f32x4 v4 = {acc[d][4 * w], acc[d][4 * w + 1], acc[d][4 * w + 2], acc[d][4 * w + 3]};
-        *p = *p + v4 * a.scale;
+        grad4(a.dq, a.dq16, a.init, qi + 32 * d + 8 * w + 4 * hh, v4 * a.scale);
       }
   }
 }
@@ -506,7 +508,8 @@ __global__ __launch_bounds__(64 * KW * QS, 2) void dkdv128_kernel(Bwd128Args a) 
   const bool any_valid_key = kp_wg_first < a.valid && k0 < a.Nk;
   const int ntq = any_valid_key ? (a.Nq - qstart + kKvBM - 1) / kKvBM : 0;
   const int nsteps = ntq * a.group;
-  if (nsteps == 0) return;  // no visible (query, key) pair: no contribution
+  // No visible (query, key) pair: no contribution (but every row may have to be written).
+  if (nsteps == 0 && !a.init && a.dk16 == nullptr) return;
   // Group g takes the steps g, g + QS, ...; every group passes every barrier.
   const int niter = QS == 1 ? nsteps : (nsteps + QS - 1) / QS;
 
@@ -525,11 +528,11 @@ __global__ __launch_bounds__(64 * KW * QS, 2) void dkdv128_kernel(Bwd128Args a) 
   };
   // The group's first step: (head, query tile) number grp of the walk.
   int hq0 = hk * a.group, qfirst = qstart;
-  if constexpr (QS > 1) {
+  if (QS > 1 && ntq > 0) {
     hq0 += grp / ntq;
     qfirst += grp % ntq * kKvBM;
   }
-  if (QS == 1 || grp < nsteps) issue(hq0, qfirst, 0);
+  if (grp < nsteps) issue(hq0, qfirst, 0);
 
   // K^T as the B operand in VGPRs: lane l holds key kw0 + l%32, dims 16t + 8h .. +7.
   bf16x8 kreg[D / 16];
@@ -720,7 +723,7 @@ __global__ __launch_bounds__(64 * KW * QS, 2) void dkdv128_kernel(Bwd128Args a) 
         ++hq;
       }
     } else {
-      while (q >= qstart + ntq * kKvBM) {
+      while (ntq > 0 && q >= qstart + ntq * kKvBM) {
         q -= ntq * kKvBM;
         ++hq;
       }
@@ -790,18 +793,16 @@ __global__ __launch_bounds__(64 * KW * QS, 2) void dkdv128_kernel(Bwd128Args a) 
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           const int d0 = 32 * dblk + 8 * w + 4 * h;
-          f32x4* pk = reinterpret_cast<f32x4*>(a.dk + off + d0);
-          f32x4* pv = reinterpret_cast<f32x4*>(a.dv + off + d0);
           const f32x4 k4 = {dk[dblk][4 * w], dk[dblk][4 * w + 1], dk[dblk][4 * w + 2], dk[dblk][4 * w + 3]};
           const f32x4 v4 = {dv[dblk][4 * w], dv[dblk][4 * w + 1], dv[dblk][4 * w + 2], dv[dblk][4 * w + 3]};
-          *pk = *pk + k4 * a.scale;
-          *pv = *pv + v4;
+          grad4(a.dk, a.dk16, a.init, off + d0, k4 * a.scale);
+          grad4(a.dv, a.dv16, a.init, off + d0, v4);
         }
     }
   } else {
     // The groups' partials meet in LDS, dK first, then dV.
     float* part = reinterpret_cast<float*>(smem);
-    auto reduce = [&](const f32x16 (&acc)[4], float* out, float scale) {
+    auto reduce = [&](const f32x16 (&acc)[4], float* dst, uint16_t* out, float scale) {
       __syncthreads();  // the tiles, or the previous partials, are done with
       float* prow = part + (wave_wg * kKvKW + kc) * kPartPitch + 4 * h;
 #pragma unroll
@@ -819,12 +820,12 @@ __global__ __launch_bounds__(64 * KW * QS, 2) void dkdv128_kernel(Bwd128Args a) 
 #pragma unroll
         for (int g = 1; g < QS; ++g)
           sum += *reinterpret_cast<const f32x4*>(part + (g * kKvBN + key) * kPartPitch + d);
-        f32x4* p = reinterpret_cast<f32x4*>(out + (((int64_t)b * a.k_rows + k0 + key) * a.Hkv + hk) * D + d);
-        *p = *p + sum * scale;
+        grad4(dst, out, a.init, (((int64_t)b * a.k_rows + k0 + key) * a.Hkv + hk) * D + d,
+              sum * scale);
       }
     };
-    reduce(dk, a.dk, a.scale);
-    reduce(dv, a.dv, 1.f);
+    reduce(dk, a.dk, a.dk16, a.scale);
+    reduce(dv, a.dv, a.dv16, 1.f);
   }
 }
 
@@ -854,6 +855,8 @@ Bwd128Args make_args(const Problem& p, const void* q, const void* k, const void*
   a.scale = p.scale;
   a.ds = nullptr;
   a.ds_nqt = a.ds_nkb = 0;
+  a.init = 0;
+  a.dq16 = a.dk16 = a.dv16 = nullptr;
   return a;
 }
 
@@ -861,9 +864,11 @@ Bwd128Args make_args(const Problem& p, const void* q, const void* k, const void*
 
 hipError_t launch_dq128(const Problem& p, const void* q, const void* k, const void* v,
                         const void* dout, const float* lse2, const float* delta, float* dq,
-                        hipStream_t s, int64_t k_rows) {
+                        hipStream_t s, int64_t k_rows, const Sink& to) {
   if (p.D != D) return hipErrorInvalidValue;
   Bwd128Args a = make_args(p, q, k, v, dout, lse2, delta);
+  a.init = to.init;
+  a.dq16 = to.out;
   if (k_rows >= 0) a.k_rows = k_rows;
   a.dq = dq;
   a.n_tiles = (p.Nq + kDqBM - 1) / kDqBM;
@@ -873,9 +878,13 @@ hipError_t launch_dq128(const Problem& p, const void* q, const void* k, const vo
 
 hipError_t launch_dkdv128(const Problem& p, const void* q, const void* k, const void* v,
                           const void* dout, const float* lse2, const float* delta, float* dk,
-                          float* dv, hipStream_t s, int64_t q_rows, uint16_t* ds) {
+                          float* dv, hipStream_t s, int64_t q_rows, uint16_t* ds,
+                          const Sink& to) {
   if (p.D != D) return hipErrorInvalidValue;
   Bwd128Args a = make_args(p, q, k, v, dout, lse2, delta);
+  a.init = to.init;
+  a.dk16 = to.out;
+  a.dv16 = to.out2;
   if (q_rows >= 0) a.q_rows = q_rows;
   a.dk = dk;
   a.dv = dv;
@@ -906,9 +915,12 @@ hipError_t launch_dkdv128(const Problem& p, const void* q, const void* k, const 
 }
 
 hipError_t launch_dqds128(const Problem& p, const void* k, const uint16_t* ds, int ds_nqt,
-                          int ds_nkb, float* dq, hipStream_t s, int64_t k_rows, int64_t q_rows) {
+                          int ds_nkb, float* dq, hipStream_t s, int64_t k_rows, int64_t q_rows,
+                          const Sink& to) {
   if (p.D != D) return hipErrorInvalidValue;
   Bwd128Args a = make_args(p, nullptr, k, nullptr, nullptr, nullptr, nullptr);
+  a.init = to.init;
+  a.dq16 = to.out;
   if (k_rows >= 0) a.k_rows = k_rows;
   if (q_rows >= 0) a.q_rows = q_rows;
   a.dq = dq;

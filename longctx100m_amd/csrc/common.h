@@ -142,6 +142,31 @@ __device__ __forceinline__ MergeW merge_weights(float ma, float la, float mb, fl
   return w;
 }
 
+// Four consecutive results r to fp32 dst, or, when out is set, rounded to bf16
+// there instead (dst and out at the same element; out 8-byte aligned).
+__device__ __forceinline__ void store4(float* dst, uint16_t* out, const f32x4& r) {
+  if (out != nullptr)
+    *reinterpret_cast<uint2*>(out) =
+        make_uint2((uint32_t)f32_to_bf16(r[0]) | ((uint32_t)f32_to_bf16(r[1]) << 16),
+                   (uint32_t)f32_to_bf16(r[2]) | ((uint32_t)f32_to_bf16(r[3]) << 16));
+  else
+    *reinterpret_cast<f32x4*>(dst) = r;
+}
+
+// A gradient contribution v at element i: added to the accumulator, or (init)
+// taking its place; the sum goes to the accumulator or (out) as bf16 to out.
+__device__ __forceinline__ void grad4(float* acc, uint16_t* out, int init, int64_t i,
+                                      const f32x4& v) {
+  f32x4 r = v;
+  if (!init) r = *reinterpret_cast<const f32x4*>(acc + i) + v;
+  store4(acc + i, out != nullptr ? out + i : nullptr, r);
+}
+__device__ __forceinline__ void grad1(float* acc, uint16_t* out, int init, int64_t i, float v) {
+  const float r = init ? v : acc[i] + v;
+  if (out != nullptr) out[i] = f32_to_bf16(r);
+  else acc[i] = r;
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup p runs on
 // XCD p % 8).  Give every XCD a contiguous range of logical tile ids so the
 // tiles that share K/V (same head) share that XCD's L2.

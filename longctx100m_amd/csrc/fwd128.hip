@@ -63,6 +63,7 @@ struct Fwd128Args {
   float* o;
   float* m;
   float* l;
+  uint16_t* out;  // set: o goes here as bf16 instead (the statistics stay fp32)
   int Nq, Nk, Hq, Hkv, group, n_qtiles;
   int64_t q_pos0, k_pos0, valid;
   int64_t kv_bstride;  // elements between batches of K and V
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void fwd128_kernel(Fwd128Args a) {
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
     const float ltrue = lt > 0.f ? lt * fast_exp2(mrun - mtrue) : 0.f;
     const float mnat = (mtrue == -INFINITY) ? -INFINITY : mtrue * kLn2;
-    float* orow = a.o + (((int64_t)b * a.Nq + row) * a.Hq + hq) * D;
+    const int64_t oi = (((int64_t)b * a.Nq + row) * a.Hq + hq) * D;
     const int64_t si = ((int64_t)b * a.Hq + hq) * a.Nq + row;
     float wa = 0.f, wb = inv, mo = mnat, lo = ltrue;
     if (a.accumulate) {
@@ -338,9 +339,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void fwd128_kernel(Fwd128Args a) {
     for (int d = 0; d < 4; ++d)
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        f32x4* dst = reinterpret_cast<f32x4*>(orow + 32 * d + 8 * w + 4 * hh);
-        const f32x4 v4 = {o[d][4 * w], o[d][4 * w + 1], o[d][4 * w + 2], o[d][4 * w + 3]};
-        *dst = a.accumulate ? *dst * wa + v4 * wb : v4 * wb;
+        float* dst = a.o + oi + 32 * d + 8 * w + 4 * hh;
+        f32x4 r = f32x4{o[d][4 * w], o[d][4 * w + 1], o[d][4 * w + 2], o[d][4 * w + 3]} * wb;
+        if (a.accumulate) r = *reinterpret_cast<const f32x4*>(dst) * wa + r;
+        store4(dst, a.out != nullptr ? a.out + (dst - a.o) : nullptr, r);
       }
     if (hh == 0) {
       a.m[si] = mo;
@@ -356,7 +358,8 @@ template <int S>
 __global__ __launch_bounds__(256) void merge_splits_kernel(int64_t rows, int splits, int N, int H,
                                                            const float* po, const float* pm,
                                                            const float* pl, float* o, float* m,
-                                                           float* l, int accumulate) {
+                                                           float* l, int accumulate,
+                                                           uint16_t* out) {
   const int64_t row = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);  // (b, n, h) of o
   if (row >= rows) return;
   const int d = 4 * (threadIdx.x & 31);
@@ -385,15 +388,15 @@ __global__ __launch_bounds__(256) void merge_splits_kernel(int64_t rows, int spl
     acc += x[s] * w;
   }
   const float inv = L > 0.f ? 1.f / L : 0.f;
-  f32x4* dst = reinterpret_cast<f32x4*>(o + row * D + d);
+  float* dst = o + row * D + d;
+  f32x4 r = acc * inv;
   if (accumulate) {
     const MergeW w = merge_weights(m[si], l[si], M, L);
-    *dst = *dst * w.wa + acc * (inv * w.wb);
+    r = *reinterpret_cast<const f32x4*>(dst) * w.wa + acc * (inv * w.wb);
     M = w.m;
     L = w.l;
-  } else {
-    *dst = acc * inv;
   }
+  store4(dst, out != nullptr ? out + row * D + d : nullptr, r);
   if (d == 0) {  // the row's threads are in one wave: all have read the old statistics
     m[si] = M;
     l[si] = L;
@@ -455,7 +458,8 @@ size_t fwd128_split_bytes(const Problem& p) {
 }
 
 hipError_t launch_fwd128_split(const Problem& p, const void* q, const void* k, const void* v,
-                               float* o, float* m, float* l, void* ws, hipStream_t st) {
+                               float* o, float* m, float* l, void* ws, hipStream_t st,
+                               uint16_t* out) {
   if (p.D != D) return hipErrorInvalidValue;
   const int S = fwd128_splits(p);
   const int64_t rows = (int64_t)p.B * p.Nq * p.Hq;
@@ -474,7 +478,7 @@ hipError_t launch_fwd128_split(const Problem& p, const void* q, const void* k, c
   if (e != hipSuccess) return e;
   auto merge = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, st, rows, a.splits,
-                       p.Nq, p.Hq, po, pm, pl, o, m, l, p.accumulate ? 1 : 0);
+                       p.Nq, p.Hq, po, pm, pl, o, m, l, p.accumulate ? 1 : 0, out);
   };
   if (a.splits <= 4) merge(merge_splits_kernel<4>);
   else if (a.splits <= 8) merge(merge_splits_kernel<8>);
@@ -483,10 +487,12 @@ hipError_t launch_fwd128_split(const Problem& p, const void* q, const void* k, c
 }
 
 hipError_t launch_fwd128(const Problem& p, const void* q, const void* k, const void* v, float* o,
-                         float* m, float* l, hipStream_t s, int64_t kv_rows, bool accumulate) {
+                         float* m, float* l, hipStream_t s, int64_t kv_rows, bool accumulate,
+                         uint16_t* out) {
   if (p.D != D) return hipErrorInvalidValue;
   Fwd128Args a = make_args(p, q, k, v, o, m, l, kv_rows);
   a.accumulate = accumulate ? 1 : 0;
+  a.out = out;
   const dim3 grid(a.n_qtiles * p.Hq * p.B);
   if (no_diagonal(p)) hipLaunchKernelGGL((fwd128_kernel<8, false>), grid, dim3(512), 0, s, a);
   else hipLaunchKernelGGL((fwd128_kernel<4, false>), grid, dim3(256), 0, s, a);

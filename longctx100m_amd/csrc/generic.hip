@@ -63,6 +63,8 @@ struct GenArgs {
   int vec;         // rows can be loaded in vectors of up to four elements
   int split;       // waves of a workgroup that share its stationary rows (forward, dQ)
   float scale;
+  int init;                      // backward: replace the accumulators' contents
+  uint16_t *out, *dk16, *dv16;   // set: o (dQ), dK, dV go here as bf16 instead
 };
 
 __device__ __forceinline__ f32x4 mfma16x16x4(float a, float b, const f32x4& c) {
@@ -352,7 +354,7 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void fwd_generic_kernel(GenArgs
         lt += s < a.split ? x : 0.f;
       }
       const float den = lt > kFltMin ? lt : kFltMin;
-      float* orow = a.o + (((int64_t)b * a.Nq + row) * a.Hq + h) * D;
+      const int64_t oi = (((int64_t)b * a.Nq + row) * a.Hq + h) * D;
       const int64_t si = ((int64_t)b * a.Hq + h) * a.Nq + row;
       MergeW w{};
       if (a.accumulate) w = merge_weights(a.m[si], a.l[si], M, lt);
@@ -363,7 +365,9 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void fwd_generic_kernel(GenArgs
           const float x = smem[(p0 + min(s, a.split - 1)) * kPart + r * part_pitch(DP) + d];
           acc += s < a.split ? x : 0.f;
         }
-        orow[d] = a.accumulate ? orow[d] * w.wa + (acc / den) * w.wb : acc / den;
+        const float r = a.accumulate ? a.o[oi + d] * w.wa + (acc / den) * w.wb : acc / den;
+        if (a.out != nullptr) a.out[oi + d] = f32_to_bf16(r);
+        else a.o[oi + d] = r;
       }
       if (lane == 0) {
         a.m[si] = a.accumulate ? w.m : M;
@@ -407,7 +411,7 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dq_generic_kernel(GenArgs 
 
   const int q0 = qt * rows_wg + qsub * 16;
   const int kend_wg = visible_keys(a, min(qt * rows_wg + rows_wg, a.Nq) - 1);
-  if (kend_wg == 0) return;  // nothing visible: dQ gets no contribution
+  if (kend_wg == 0 && !a.init && a.out == nullptr) return;  // nothing visible: no contribution
   f32x4 qr[NJ], dor[NJ], acc[NJ];
   load_rows<T, NJ>(qr, qb, qs, q0, a.Nq, D, vec, c, g);
   load_rows<T, NJ>(dor, ob, qs, q0, a.Nq, D, vec, c, g);
@@ -451,7 +455,7 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dq_generic_kernel(GenArgs 
   for (int r = ksub; r < 16; r += a.split) {
     const int row = q0 + r;
     if (row >= a.Nq) break;
-    float* dst = a.dq + (((int64_t)b * a.Nq + row) * a.Hq + h) * D;
+    const int64_t qi = (((int64_t)b * a.Nq + row) * a.Hq + h) * D;
     for (int d = lane; d < D; d += 64) {
       float sum = 0.f;
 #pragma unroll
@@ -459,7 +463,7 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dq_generic_kernel(GenArgs 
         const float x = smem[(qsub * a.split + min(s, a.split - 1)) * kPart + r * part_pitch(DP) + d];
         sum += s < a.split ? x : 0.f;
       }
-      dst[d] += sum * a.scale;
+      grad1(a.dq, a.out, a.init, qi + d, sum * a.scale);
     }
   }
 }
@@ -513,7 +517,7 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dkdv_generic_kernel(GenArg
   }
   qstart = qstart / 16 * 16;
   const int ntq = kp_first < a.valid ? (a.Nq - qstart + 15) / 16 : 0;
-  if (ntq <= 0) return;  // no visible pair: no contribution
+  if (ntq <= 0 && !a.init && a.dk16 == nullptr) return;  // no visible pair: no contribution
   const int nsteps = ntq * a.group;
   // First query that sees the lane's key.
   int rmin = 0;
@@ -589,11 +593,11 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dkdv_generic_kernel(GenArg
   }
 
   // Sum of the waves' partials; thread (row, dims) of the workgroup.
-  auto reduce = [&](const f32x4 (&acc)[NJ], float* dst, float scale) {
+  auto reduce = [&](const f32x4 (&acc)[NJ], float* dst, uint16_t* out, float scale) {
     store_part<NJ>(smem + wave * kPart, acc, c, g);
     __syncthreads();
     for (int r = wave; r < 16 && k0 + r < a.Nk; r += nw) {
-      float* out = dst + (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D;
+      const int64_t ki = (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D;
       for (int d = lane; d < D; d += 64) {
         float sum = 0.f;
 #pragma unroll
@@ -601,14 +605,14 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dkdv_generic_kernel(GenArg
           const float x = smem[min(w, nw - 1) * kPart + r * part_pitch(DP) + d];
           sum += w < nw ? x : 0.f;
         }
-        out[d] += sum * scale;
+        grad1(dst, out, a.init, ki + d, sum * scale);
       }
     }
   };
   if constexpr (kKvLds) __syncthreads();  // every wave is done with K and V
-  reduce(dk, a.dk, a.scale);
+  reduce(dk, a.dk, a.dk16, a.scale);
   __syncthreads();
-  reduce(dv, a.dv, 1.f);
+  reduce(dv, a.dv, a.dv16, 1.f);
 }
 
 // Waves the chip holds at two per SIMD, the occupancy of these kernels.
@@ -671,9 +675,10 @@ void dispatch(const Problem& p, const F& f) {
 }  // namespace
 
 hipError_t launch_fwd_generic(const Problem& p, const void* q, const void* k, const void* v,
-                              float* o, float* m, float* l, hipStream_t s) {
+                              float* o, float* m, float* l, hipStream_t s, uint16_t* out) {
   if (p.D > 256) return hipErrorInvalidValue;
   GenArgs a = make_args(p, q, k, v, nullptr);
+  a.out = out;
   a.o = o;
   a.m = m;
   a.l = l;
@@ -699,9 +704,11 @@ hipError_t launch_fwd_generic(const Problem& p, const void* q, const void* k, co
 
 hipError_t launch_bwd_dq_generic(const Problem& p, const void* q, const void* k, const void* v,
                                  const void* dout, const float* lse2, const float* delta,
-                                 float* dq, hipStream_t s) {
+                                 float* dq, hipStream_t s, const Sink& to) {
   if (p.D > 256) return hipErrorInvalidValue;
   GenArgs a = make_args(p, q, k, v, dout);
+  a.init = to.init;
+  a.out = to.out;
   a.lse2 = lse2;
   a.delta = delta;
   a.dq = dq;
@@ -721,9 +728,12 @@ hipError_t launch_bwd_dq_generic(const Problem& p, const void* q, const void* k,
 
 hipError_t launch_bwd_dkdv_generic(const Problem& p, const void* q, const void* k, const void* v,
                                    const void* dout, const float* lse2, const float* delta,
-                                   float* dk, float* dv, hipStream_t s) {
+                                   float* dk, float* dv, hipStream_t s, const Sink& to) {
   if (p.D > 256) return hipErrorInvalidValue;
   GenArgs a = make_args(p, q, k, v, dout);
+  a.init = to.init;
+  a.dk16 = to.out;
+  a.dv16 = to.out2;
   a.lse2 = lse2;
   a.delta = delta;
   a.dk = dk;

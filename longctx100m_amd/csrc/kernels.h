@@ -19,6 +19,16 @@ struct Problem {
   bool accumulate;  // forward: LSE-merge into the running (o, m, l) instead of writing them
 };
 
+// Where the results of a launch go.  init (backward): the contribution takes
+// the place of what the accumulator holds, which need not be initialised, and
+// every row is written; out: the results go here as bf16 (dk and dv: the
+// second pointer for dv) instead of the fp32 buffer.
+struct Sink {
+  bool init = false;
+  uint16_t* out = nullptr;
+  uint16_t* out2 = nullptr;
+};
+
 // Index of the exclusive end of the keys that any query of [q_begin, q_end)
 // can see, clipped to [0, Nk].
 inline int64_t key_end_for(const Problem& p, int64_t q_end) {
@@ -43,7 +53,7 @@ bool mfma_supported(const Problem& p);
 // launch_fwd_generic take it from p.accumulate).
 hipError_t launch_fwd128(const Problem& p, const void* q, const void* k, const void* v, float* o,
                          float* m, float* l, hipStream_t s, int64_t kv_rows = -1,
-                         bool accumulate = false);
+                         bool accumulate = false, uint16_t* out = nullptr);
 // Small grids: the keys in up to kFwdMaxSplits splits of at least
 // kFwdSplitKeys, as many as the chip holds workgroups for, whose partials lie in a workspace
 // of fwd128_split_bytes (0: one split) and are merged by a second kernel.
@@ -52,17 +62,19 @@ constexpr int64_t kFwdSplitKeys = 512;
 int fwd128_splits(const Problem& p);
 size_t fwd128_split_bytes(const Problem& p);
 hipError_t launch_fwd128_split(const Problem& p, const void* q, const void* k, const void* v,
-                               float* o, float* m, float* l, void* ws, hipStream_t s);
+                               float* o, float* m, float* l, void* ws, hipStream_t s,
+                               uint16_t* out = nullptr);
 // The backward can run on a sub-shard too (results accumulate into dq, dk,
 // dv anyway): dQ on a key sub-shard (k, v at its first key, k_rows = keys of
 // the whole shard), dK/dV on a query sub-shard (q, dout, lse2, delta at its
 // first query, q_rows = queries of the whole shard).  -1: p's own count.
 hipError_t launch_dq128(const Problem& p, const void* q, const void* k, const void* v,
                         const void* dout, const float* lse2, const float* delta, float* dq,
-                        hipStream_t s, int64_t k_rows = -1);
+                        hipStream_t s, int64_t k_rows = -1, const Sink& to = {});
 hipError_t launch_dkdv128(const Problem& p, const void* q, const void* k, const void* v,
                           const void* dout, const float* lse2, const float* delta, float* dk,
-                          float* dv, hipStream_t s, int64_t q_rows = -1, uint16_t* ds = nullptr);
+                          float* dv, hipStream_t s, int64_t q_rows = -1, uint16_t* ds = nullptr,
+                          const Sink& to = {});
 // dS sharing: launch_dkdv128 with ds set also writes every dS block it forms
 // (ceil(Nq/32) x ceil(Nk/32) blocks of 2 KB per (batch, query head), layout
 // in bwd128.hip); launch_dqds128 then adds dQ = scale dS K from those blocks
@@ -72,26 +84,27 @@ hipError_t launch_dkdv128(const Problem& p, const void* q, const void* k, const 
 constexpr size_t kDsBlockBytes = 2048;
 hipError_t launch_dqds128(const Problem& p, const void* k, const uint16_t* ds, int ds_nqt,
                           int ds_nkb, float* dq, hipStream_t s, int64_t k_rows = -1,
-                          int64_t q_rows = -1);
+                          int64_t q_rows = -1, const Sink& to = {});
 
 // head_dim 64 (attn64.hip).
 hipError_t launch_fwd64(const Problem& p, const void* q, const void* k, const void* v, float* o,
-                        float* m, float* l, hipStream_t s);
+                        float* m, float* l, hipStream_t s, uint16_t* out = nullptr);
 hipError_t launch_dq64(const Problem& p, const void* q, const void* k, const void* v,
                        const void* dout, const float* lse2, const float* delta, float* dq,
-                       hipStream_t s);
+                       hipStream_t s, const Sink& to = {});
 hipError_t launch_dkdv64(const Problem& p, const void* q, const void* k, const void* v,
                          const void* dout, const float* lse2, const float* delta, float* dk,
-                         float* dv, hipStream_t s);
+                         float* dv, hipStream_t s, const Sink& to = {});
 hipError_t launch_fwd_generic(const Problem& p, const void* q, const void* k, const void* v,
-                              float* o, float* m, float* l, hipStream_t s);
+                              float* o, float* m, float* l, hipStream_t s,
+                              uint16_t* out = nullptr);
 
 hipError_t launch_bwd_dq_generic(const Problem& p, const void* q, const void* k, const void* v,
                                  const void* dout, const float* lse2, const float* delta,
-                                 float* dq, hipStream_t s);
+                                 float* dq, hipStream_t s, const Sink& to = {});
 hipError_t launch_bwd_dkdv_generic(const Problem& p, const void* q, const void* k, const void* v,
                                    const void* dout, const float* lse2, const float* delta,
-                                   float* dk, float* dv, hipStream_t s);
+                                   float* dk, float* dv, hipStream_t s, const Sink& to = {});
 
 // Row-wise helpers.  rows = B * N * H, row r = ((b * N) + t) * H + h.
 hipError_t launch_merge(int B, int N, int H, int D, float* o_run, float* m_run, float* l_run,
