@@ -312,8 +312,9 @@ __device__ __forceinline__ int ds_query(int j) {
   return 16 * (c >> 3) + 4 * cb + ((c >> 2) & 1) + 2 * (c & 1) + 8 * ((c >> 1) & 1);
 }
 
-// LDS: K double-buffered and dS in kDsStages buffers, both one tile ahead (the
-// dS stream comes from HBM): 160 KB, one workgroup per CU.
+// LDS: K double-buffered, one tile ahead, and dS in kDsStages buffers (the dS
+// stream comes from HBM).  Sixteen waves: dS one tile ahead, 160 KB, one
+// workgroup per CU.  Four waves (small grids): dS two tiles ahead, 80 KB.
 template <int kDsNW>
 __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
   constexpr int kDsBM = kDsNW * kDqQW;  // queries per workgroup
