@@ -462,25 +462,7 @@ int lc_attn_decode_static(const lc_attn_shape_t* shape, const lc_attn_mask_t* ma
     return fwd_shard(p, q, k, v, o, m, l, st);  // the blockwise kernels use no scratch
   const size_t need = round_up(lc::decode_workspace_bytes(p));
   if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
-  if (need > lc::kDecodeStaticScratchBytes && !lc::decode_workspace_required(p))
-    return fwd_shard(p, q, k, v, o, m, l, st);
+    return fwd_shard(p, q, k, v, o, m, l, st);  // may do without a workspace
   if (need > lc::kDecodeStaticScratchBytes)
     return set_error(LC_ERR_WORKSPACE,
                      "decode needs %zu bytes of scratch, more than the static maximum of %zu; "
