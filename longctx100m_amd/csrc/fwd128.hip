@@ -382,8 +382,9 @@ __global__ __launch_bounds__(256) void merge_splits_kernel(int64_t rows, int spl
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    if (ms[s] == -INFINITY) continue;  // the split saw no key
-    const float w = expf(ms[s] - M) * ls[s];
+    if (s >= splits) continue;
+    // No key seen (x is zeros), or NaN scores only (x is NaN and has to stay so).
+    const float w = ms[s] == -INFINITY ? 0.f : expf(ms[s] - M) * ls[s];
     L += w;
     acc += x[s] * w;
   }

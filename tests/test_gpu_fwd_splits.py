@@ -66,6 +66,35 @@ def test_fwd_splits(gpu, case):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("where", ["query", "key"])
+def test_nan_passes_through_the_splits(gpu, where):
+    """A NaN query leaves every split of its row without a maximum: the row is
+    NaN as in the unsplit call, not zeros; a NaN key reaches the rows that see it."""
+    from longctx100m_amd import ring_attention as ra
+
+    nq, nk = 33, 2100
+    q, k, v = (gpu.randn(1, n, 2, 128, device="cuda").to(gpu.bfloat16) for n in (nq, nk, nk))
+    if where == "query":
+        q[0, 7, 1] = float("nan")
+    else:
+        k[0, 2090, 1, 5] = float("nan")
+    mk = _lib.Mask(nk - nq, 0, -1, 1, 0)
+    o, m, l = ra.fwd_shard(q, k, v, q_pos0=nk - nq, k_pos0=0)
+    o1, m1, l1 = (gpu.zeros_like(t) for t in (o, m, l))
+    _lib.check(_lib.load().lc_attn_fwd_shard(
+        _lib.Shape(1, nq, nk, 2, 2, 128, _lib.LC_DTYPE_BF16, 0), mk,
+        *(t.data_ptr() for t in (q, k, v, o1, m1, l1)), gpu.cuda.current_stream().cuda_stream))
+    want = gpu.zeros(nq, 2, dtype=gpu.bool)
+    if where == "query":
+        want[7, 1] = True
+    else:
+        want[2090 - (nk - nq):, 1] = True
+    for t in (o, o1):
+        assert gpu.equal(t[0].isnan().all(-1).cpu(), want)
+        assert gpu.equal(t[0].isnan().any(-1).cpu(), want)
+
+
+@pytest.mark.gpu
 def test_ring_forward_with_the_least_workspace(gpu):
     """lc_ring_fwd_with_stats takes the running output alone as its workspace and
     then runs its hops unsplit."""
