@@ -145,6 +145,15 @@ __global__ __launch_bounds__(64 * W, NB * W == 1 ? 1 : 2) void decode_kernel(Dec
   using C = DecodeTile<D>;
   constexpr int TK = C::TK, MB = C::MB, KS = C::KS, DB = C::DB;
   constexpr int kRows = 16 * NB;
+  // head_dim 128, one row block: the probabilities that are rounded to bf16
+  // are relative to their own tile's maximum, and the tile's product joins the
+  // fp32 state with an fp32 weight.  Each tile's largest probability is then
+  // exact; relative to a maximum that runs over the four tiles of a wave the
+  // outputs were further from 64 bits (500 keys x 32/8 heads: 1.3e-3 against
+  // 1.1e-3 here).  The kernel waits for memory: the 64 multiplications more per
+  // tile leave that call at 14.4 us.  Long single streams (W = 1) keep the
+  // running maximum: 1.4e-3 either way.
+  constexpr bool kTileRef = TK == 32 && NB == 1 && W > 1;
   constexpr int kPitch = D + 4;  // floats per row of a wave's partial
   constexpr int kVBytes = W * kStages * kTileBytes;
   constexpr int kPartBytes = W * kRows * kPitch * 4;
@@ -257,6 +266,7 @@ __global__ __launch_bounds__(64 * W, NB * W == 1 ? 1 : 2) void decode_kernel(Dec
     const int key0 = (int)(kb0 + (int64_t)j * (W * TK));
     const int kmax = (int)min((int64_t)TK, kb1 - key0);  // keys of this tile inside the workgroup's share
 
+    float alpha = 1.f, beta = 1.f;  // kTileRef: weights of the state and of the tile
     f32x4 sc[NB][MB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
@@ -281,22 +291,31 @@ __global__ __launch_bounds__(64 * W, NB * W == 1 ? 1 : 2) void decode_kernel(Dec
           mx = fmaxf(mx, sc[nb][mb][i]);
         }
       mx = group4_max(mx);
-      if (mx > mrow[nb]) {
-        const float alpha = fast_exp2(mrow[nb] - mx);  // mrow = -inf: 0
-        lsum[nb] *= alpha;
+      if constexpr (kTileRef) {
+        const float mnew = fmaxf(mrow[nb], mx);
+        alpha = mrow[nb] == -INFINITY ? 0.f : fast_exp2(mrow[nb] - mnew);
+        beta = mx == -INFINITY ? 0.f : fast_exp2(mx - mnew);
+        mrow[nb] = mnew;
+      } else if (mx > mrow[nb]) {
+        const float up = fast_exp2(mrow[nb] - mx);  // mrow = -inf: 0
+        lsum[nb] *= up;
 #pragma unroll
-        for (int db = 0; db < DB; ++db) o[nb][db] *= alpha;
+        for (int db = 0; db < DB; ++db) o[nb][db] *= up;
         mrow[nb] = mx;
       }
-      const float muse = mrow[nb] == -INFINITY ? 0.f : mrow[nb];  // no key yet: p = 0
+      const float ref = kTileRef ? mx : mrow[nb];
+      const float muse = ref == -INFINITY ? 0.f : ref;  // no key yet: p = 0
+      float tsum = 0.f;
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float p = fast_exp2(sc[nb][mb][i] - muse);
-          lsum[nb] += p;
+          if constexpr (kTileRef) tsum += p;
+          else lsum[nb] += p;
           sc[nb][mb][i] = p;
         }
+      if constexpr (kTileRef) lsum[nb] = lsum[nb] * alpha + tsum * beta;
     }
 #pragma unroll
     for (int k2 = 0; k2 < TK / 32; ++k2) {
@@ -308,7 +327,12 @@ __global__ __launch_bounds__(64 * W, NB * W == 1 ? 1 : 2) void decode_kernel(Dec
         const uint8_t* p = vt + voff[db] + 32 * k2 * 2 * D;
         const bf16x8 va = concat_bf16x4(t128::ds_read_tr(p), t128::ds_read_tr(p + 16 * 2 * D));
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) o[nb][db] = mfma16x16x32(va, pb[nb], o[nb][db]);
+        for (int nb = 0; nb < NB; ++nb) {
+          if constexpr (kTileRef)
+            o[nb][db] = o[nb][db] * alpha + mfma16x16x32(va, pb[nb], f32x4{0.f, 0.f, 0.f, 0.f}) * beta;
+          else
+            o[nb][db] = mfma16x16x32(va, pb[nb], o[nb][db]);
+        }
       }
     }
   };

@@ -25,6 +25,8 @@ CASES = [
     (1, 16, 1500, 4, 1, 128, -900, 0, True, None),      # 64 rows, queries inside the cache
     (1, 8, 16001, 8, 2, 128, 0, 0, True, None),         # 32 rows over many splits
     (1, 3, 40, 4, 4, 128, -39, 7, True, None),          # rows that see few keys, splits without any
+    (1, 1, 500, 32, 8, 128, 0, 0, True, None),          # four tiles for each wave, one split
+    (2, 4, 1000, 8, 2, 128, -500, 0, True, 700),        # tiles without a visible key after others
     (1, 1, 300000, 2, 1, 64, 0, 0, False, None),        # a long single stream: one-wave workgroups
     (1, 20, 140000, 1, 1, 128, 0, 0, True, 139000),     # the same with 32 rows
     (33, 1, 70, 16, 16, 64, 0, 0, True, None),          # more heads than the chip holds at once
