@@ -574,7 +574,7 @@ int decode_splits(const Problem& p) {
 }
 
 bool decode_supported(const Problem& p) {
-  return p.dtype == 1 && !p.precise && (p.D == 64 || p.D == 128) &&
+  return p.dtype == 1 && !p.precise && (p.D == 64 || p.D == 128) && p.Nq > 0 &&
          (int64_t)p.Nq * (p.Hq / p.Hkv) <= kDecodeMaxRows;
 }
 

@@ -118,7 +118,7 @@ hipError_t launch_bwd_preprocess(int B, int N, int H, int D, int dtype, const vo
                                  const void* dout, const float* m, const float* l, float* delta,
                                  float* lse2, hipStream_t s);
 
-// Split-KV decode attention (decode.hip): bf16, D = 64 or 128, at most
+// Split-KV decode attention (decode.hip): bf16, D = 64 or 128, one to
 // kDecodeMaxRows query rows (Nq * Hq / Hkv) per KV head.
 // decode_workspace_required: a workspace of decode_workspace_bytes must be
 // given (D = 128, at most 16 rows); other shapes may run the blockwise kernels

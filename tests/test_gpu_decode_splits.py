@@ -81,3 +81,19 @@ def test_required_workspace_sizes_are_kept():
         splits = max(1, min(-(-2048 // (b * hkv)), -(-nk // 32) // 2, 4096))
         need = splits * b * nq * hq * (128 * 4 + 8)
         assert lib.lc_attn_decode_workspace_bytes(ctypes.byref(s)) == -(-need // 256) * 256
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("nk", [0, 1, 3001, 300000])
+def test_empty_queries_need_no_workspace(d, nk):
+    """No query rows: the size query answers 0 (there is nothing to split) and
+    the calls return without work, whatever the cache."""
+    lib = _lib.load()
+    mk = _lib.Mask(0, 0, -1, 1, 0)
+    for b, hq, hkv in ((1, 9, 3), (2, 8, 8), (1, 64, 1)):
+        s = _lib.Shape(b, 0, nk, hq, hkv, d, _lib.LC_DTYPE_BF16, 0)
+        assert lib.lc_attn_decode_workspace_bytes(ctypes.byref(s)) == 0
+        assert lib.lc_attn_fwd_shard_workspace_bytes(ctypes.byref(s)) == 0
+        ptrs = [256] * 6  # never read
+        assert lib.lc_attn_decode(ctypes.byref(s), ctypes.byref(mk), *ptrs, None, 0, None) == 0
+        assert lib.lc_attn_decode_static(ctypes.byref(s), ctypes.byref(mk), *ptrs, None) == 0
