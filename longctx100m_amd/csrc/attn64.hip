@@ -192,6 +192,24 @@ __device__ __forceinline__ f32x4 sum_parts(const uint8_t* smem, int wave0, int s
   return acc;
 }
 
+// The thread's rows r0, r0 + 4 split, ... < min(kRows, nrows) of a summed partial block to
+// the gradient, four rows at a time (grad_add); at(r): element of row r.
+template <int W, typename At>
+__device__ __forceinline__ void grad_rows(float* dst, uint16_t* out, int init, int split, int r0,
+                                          int nrows, const At& at, const uint8_t* smem, int wave0,
+                                          int off) {
+  for (int base = r0; base < kRows; base += 16 * split) {
+    f32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = min(base + 4 * split * j, kRows - 1);
+      v[j] = sum_parts<W>(smem, wave0, split, r * kPitch + off);
+    }
+    grad_add(dst, out, init, v, [&](int j) { return at(base + 4 * split * j); },
+             [&](int j) { return base + 4 * split * j < min(kRows, nrows); });
+  }
+}
+
 // ----------------------------------------------------------------- forward --
 
 // Wave w of the workgroup: query block w / split (NQ x 32 queries), key tiles
@@ -478,13 +496,11 @@ __global__ __launch_bounds__(64 * W, 2) void dq64_kernel(Args64 a) {
     if (n > 0) __syncthreads();
     store_part(reinterpret_cast<float*>(mem), acc[n], a.scale, lane);
     __syncthreads();
-    for (int r = 4 * ksub + (lane >> 4); r < kRows; r += 4 * a.split) {
-      const int row = q0 + kRows * n + r;
-      if (row >= a.Nq) break;
-      const int d = 4 * (lane & 15);
-      grad4(a.dq, a.out, a.init, (((int64_t)b * a.Nq + row) * a.Hq + h) * D + d,
-            sum_parts<W>(smem, qsub * a.split, a.split, r * kPitch + d));
-    }
+    const int r0 = 4 * ksub + (lane >> 4), d = 4 * (lane & 15);
+    grad_rows<W>(
+        a.dq, a.out, a.init, a.split, r0, a.Nq - (q0 + kRows * n),
+        [&](int r) { return (((int64_t)b * a.Nq + q0 + kRows * n + r) * a.Hq + h) * D + d; },
+        smem, qsub * a.split, d);
   }
 }
 
@@ -626,14 +642,10 @@ __global__ __launch_bounds__(64 * W, 2) void dkdv64_kernel(Args64 a) {
   store_part(reinterpret_cast<float*>(mem), dk, a.scale, lane);
   store_part(reinterpret_cast<float*>(mem) + kPart, dv, 1.f, lane);
   __syncthreads();
-  for (int r = 4 * qsub + (lane >> 4); r < kRows; r += 4 * a.split) {
-    if (k0 + r >= a.Nk) break;
-    const int d = 4 * (lane & 15);
-    const int64_t off = (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D + d;
-    grad4(a.dk, a.dk16, a.init, off, sum_parts<W>(smem, ksub * a.split, a.split, r * kPitch + d));
-    grad4(a.dv, a.dv16, a.init, off,
-          sum_parts<W>(smem, ksub * a.split, a.split, kPart + r * kPitch + d));
-  }
+  const int r0 = 4 * qsub + (lane >> 4), d = 4 * (lane & 15);
+  auto at = [&](int r) { return (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D + d; };
+  grad_rows<W>(a.dk, a.dk16, a.init, a.split, r0, a.Nk - k0, at, smem, ksub * a.split, d);
+  grad_rows<W>(a.dv, a.dv16, a.init, a.split, r0, a.Nk - k0, at, smem, ksub * a.split, kPart + d);
 }
 
 Args64 make_args(const Problem& p, const void* q, const void* k, const void* v, const void* dout) {

@@ -132,15 +132,20 @@ __global__ __launch_bounds__(256, 2) void dq128_kernel(Bwd128Args a) {
   if (a.causal) kend = min(kend, a.q_pos0 + q_end - a.k_pos0);
   kend = min(kend, a.valid - a.k_pos0);
   const int ntiles = kend > 0 ? (int)((kend + kDqBN - 1) / kDqBN) : 0;
-  if (ntiles == 0 && !a.init && a.dq16 == nullptr) return;  // nothing visible: no contribution
+  if (ntiles == 0) {  // nothing visible: no contribution (but every row may have to be written)
+    if ((a.init || a.dq16 != nullptr) && qw0 + kc < a.Nq) {
+      const f32x16 zero[4] = {};
+      grad_row(a.dq, a.dq16, a.init, (((int64_t)b * a.q_rows + qw0 + kc) * a.Hq + h) * D + 4 * hh,
+               zero, 1.f);
+    }
+    return;
+  }
 
   const uint32_t smem_lds = t128::lds_addr(smem);
   t128::RowLoader<kDqBN, 4> ld;
   ld.init(ks, wave, lane);
-  if (ntiles > 0) {
-    ld.load(kbase, ks, 0, a.Nk, smem_lds, wave, lane);
-    ld.load(vbase, ks, 0, a.Nk, smem_lds + kDqTile, wave, lane);
-  }
+  ld.load(kbase, ks, 0, a.Nk, smem_lds, wave, lane);
+  ld.load(vbase, ks, 0, a.Nk, smem_lds + kDqTile, wave, lane);
 
   // Q^T, dO^T as B operands: lane holds query qw0 + kc, dims 16t + 8hh .. +7.
   bf16x8 qreg[D / 16], doreg[D / 16];
@@ -277,13 +282,7 @@ __global__ __launch_bounds__(256, 2) void dq128_kernel(Bwd128Args a) {
   const int row = qw0 + kc;
   if (row < a.Nq) {
     const int64_t qi = (((int64_t)b * a.q_rows + row) * a.Hq + h) * D;
-#pragma unroll
-    for (int d = 0; d < 4; ++d)
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const f32x4 v4 = {acc[d][4 * w], acc[d][4 * w + 1], acc[d][4 * w + 2], acc[d][4 * w + 3]};
-        grad4(a.dq, a.dq16, a.init, qi + 32 * d + 8 * w + 4 * hh, v4 * a.scale);
-      }
+    grad_row(a.dq, a.dq16, a.init, qi + 4 * hh, acc, a.scale);
   }
 }
 
@@ -438,13 +437,7 @@ __global__ __launch_bounds__(64 * kDsNW, 1) void dqds128_kernel(Bwd128Args a) {
   const int row = qw0 + ds_query(kc);
   if ((nt_w > 0 || a.init || a.dq16 != nullptr) && row < a.Nq) {
     const int64_t qi = (((int64_t)b * a.q_rows + row) * a.Hq + h) * D;
-#pragma unroll
-    for (int d = 0; d < 4; ++d)
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const f32x4 v4 = {acc[d][4 * w], acc[d][4 * w + 1], acc[d][4 * w + 2], acc[d][4 * w + 3]};
-        grad4(a.dq, a.dq16, a.init, qi + 32 * d + 8 * w + 4 * hh, v4 * a.scale);
-      }
+    grad_row<kDsNW == 16 ? 8 : 16>(a.dq, a.dq16, a.init, qi + 4 * hh, acc, a.scale);
   }
 }
 
@@ -788,17 +781,9 @@ __global__ __launch_bounds__(64 * KW * QS, 2) void dkdv128_kernel(Bwd128Args a) 
   if constexpr (QS == 1) {
     const int row = kw0 + kc;
     if (row < a.Nk) {
-      const int64_t off = (((int64_t)b * a.k_rows + row) * a.Hkv + hk) * D;
-#pragma unroll
-      for (int dblk = 0; dblk < 4; ++dblk)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const int d0 = 32 * dblk + 8 * w + 4 * h;
-          const f32x4 k4 = {dk[dblk][4 * w], dk[dblk][4 * w + 1], dk[dblk][4 * w + 2], dk[dblk][4 * w + 3]};
-          const f32x4 v4 = {dv[dblk][4 * w], dv[dblk][4 * w + 1], dv[dblk][4 * w + 2], dv[dblk][4 * w + 3]};
-          grad4(a.dk, a.dk16, a.init, off + d0, k4 * a.scale);
-          grad4(a.dv, a.dv16, a.init, off + d0, v4);
-        }
+      const int64_t off = (((int64_t)b * a.k_rows + row) * a.Hkv + hk) * D + 4 * h;
+      grad_row(a.dk, a.dk16, a.init, off, dk, a.scale);
+      grad_row(a.dv, a.dv16, a.init, off, dv, 1.f);
     }
   } else {
     // The groups' partials meet in LDS, dK first, then dV.
@@ -814,16 +799,24 @@ __global__ __launch_bounds__(64 * KW * QS, 2) void dkdv128_kernel(Bwd128Args a) 
               f32x4{acc[dblk][4 * w], acc[dblk][4 * w + 1], acc[dblk][4 * w + 2], acc[dblk][4 * w + 3]};
       __syncthreads();
       constexpr int kPer = D / 4;  // threads per key
-      for (int it = tid; it < kKvBN * kPer; it += 64 * KW * QS) {
-        const int key = it / kPer, d = 4 * (it % kPer);
-        if (k0 + key >= a.Nk) break;
-        f32x4 sum = *reinterpret_cast<const f32x4*>(part + key * kPartPitch + d);
+      constexpr int kIt = kKvBN * kPer / (64 * KW * QS);
+      const int key0 = tid / kPer, d = 4 * (tid % kPer);
+      constexpr int kStep = kKvBN / kIt;  // keys of one round
+      f32x4 v[kIt];
+#pragma unroll
+      for (int it = 0; it < kIt; ++it) {
+        const float* p = part + (key0 + it * kStep) * kPartPitch + d;
+        v[it] = *reinterpret_cast<const f32x4*>(p);
 #pragma unroll
         for (int g = 1; g < QS; ++g)
-          sum += *reinterpret_cast<const f32x4*>(part + (g * kKvBN + key) * kPartPitch + d);
-        grad4(dst, out, a.init, (((int64_t)b * a.k_rows + k0 + key) * a.Hkv + hk) * D + d,
-              sum * scale);
+          v[it] += *reinterpret_cast<const f32x4*>(p + g * kKvBN * kPartPitch);
+        v[it] *= scale;
       }
+      grad_add(dst, out, a.init, v,
+               [&](int it) {
+                 return (((int64_t)b * a.k_rows + k0 + key0 + it * kStep) * a.Hkv + hk) * D + d;
+               },
+               [&](int it) { return k0 + key0 + it * kStep < a.Nk; });
     };
     reduce(dk, a.dk, a.dk16, a.scale);
     reduce(dv, a.dv, a.dv16, 1.f);

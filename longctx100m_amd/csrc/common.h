@@ -153,13 +153,50 @@ __device__ __forceinline__ void store4(float* dst, uint16_t* out, const f32x4& r
     *reinterpret_cast<f32x4*>(dst) = r;
 }
 
-// A gradient contribution v at element i: added to the accumulator, or (init)
-// taking its place; the sum goes to the accumulator or (out) as bf16 to out.
-__device__ __forceinline__ void grad4(float* acc, uint16_t* out, int init, int64_t i,
-                                      const f32x4& v) {
-  f32x4 r = v;
-  if (!init) r = *reinterpret_cast<const f32x4*>(acc + i) + v;
-  store4(acc + i, out != nullptr ? out + i : nullptr, r);
+// N gradient contributions v[j] at elements at(j): added to the accumulator, or
+// (init) taking its place; the sums go to the accumulator or (out) as bf16 to
+// out; on says which j exist.  The accumulator's old values are all read
+// before the first is used: with the choices made per element each read is
+// waited for by itself, which costs the kernel's end 16 memory latencies
+// instead of one (one 64-key tile, dQ of head_dim 128: 7.0 us against 4.7).
+template <int N, typename At, typename On>
+__device__ __forceinline__ void grad_add(float* acc, uint16_t* out, int init, const f32x4 (&v)[N],
+                                         const At& at, const On& on) {
+  f32x4 r[N];
+  if (init) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) r[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (on(j)) r[j] = *reinterpret_cast<const f32x4*>(acc + at(j));
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) r[j] += v[j];
+  if (out != nullptr) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (on(j)) store4(nullptr, out + at(j), r[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (on(j)) store4(acc + at(j), nullptr, r[j]);
+  }
+}
+// The same of a lane's share of a transposed 128-dim row, N vectors at a time:
+// element v of x[d] is dim 32 d + 8(v/4) + v%4 from element i on.
+template <int N = 16>
+__device__ __forceinline__ void grad_row(float* acc, uint16_t* out, int init, int64_t i,
+                                         const f32x16 (&x)[4], float scale) {
+#pragma unroll
+  for (int j0 = 0; j0 < 16; j0 += N) {
+    f32x4 v[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[j][e] = x[(j0 + j) >> 2][4 * ((j0 + j) & 3) + e] * scale;
+    grad_add(acc, out, init, v, [&](int j) { return i + 8 * (j0 + j); }, [](int) { return true; });
+  }
 }
 __device__ __forceinline__ void grad1(float* acc, uint16_t* out, int init, int64_t i, float v) {
   const float r = init ? v : acc[i] + v;
