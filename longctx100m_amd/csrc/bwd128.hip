@@ -33,6 +33,7 @@
 #include "kernels.h"
 #include "tile128.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace lc {
@@ -882,6 +883,52 @@ Bwd128Args make_args(const Problem& p, const void* q, const void* k, const void*
   return a;
 }
 
+// Keys in front of the queries, which every one of them sees (all keys without
+// a causal mask), and queries behind the keys, which see every one of them.
+int64_t keys_before(const Problem& p) {
+  return p.causal ? std::min<int64_t>(p.Nk, std::max<int64_t>(0, p.q_pos0 - p.k_pos0)) : p.Nk;
+}
+int64_t queries_after(const Problem& p) {
+  return std::max<int64_t>(0, p.q_pos0 + p.Nq - p.k_pos0 - p.Nk);
+}
+
+// dK/dV in the form whose four groups split each walk (64 keys per workgroup,
+// one per CU) instead of one walk per 128 keys (wgs workgroups, two per CU).
+// It moves each query tile into LDS for two waves instead of four, so it pays
+// where workgroups are few: up to 128 (17-64 queries over 64 keys equal, walks
+// of 16 and more steps 0.45-0.6 of the time).  Above that it pays by evening
+// out walks: up to 256 workgroups when they are long (64 steps: 0.8-1.0) or
+// when most keys lie on the diagonal (from 16 steps on: 0.6-0.95; 4,096
+// tokens, 32/8 heads 565 -> 311 us), up to 512 when all but a tenth do and
+// there are heads enough for every XCD to hold long and short walks (8,192
+// tokens, 32/8 heads 1293 -> 1144 us).  Elsewhere the walks of the whole are
+// the shorter: 512 queries over 20,000 keys, 9/3 heads (471 workgroups, a few
+// tiles each) 104 us against 158; 512 tokens, 8 x 16 heads 49 against 70; one
+// head, 60,000 keys 1.0 against 1.4.
+bool split_walks(const Problem& p, int64_t wgs, int64_t heads) {
+  const int64_t steps = (int64_t)(p.Nq + 31) / 32 * (p.Hq / p.Hkv), before = keys_before(p);
+  if (wgs <= 128) return true;
+  if (before >= p.Nk) return false;  // no diagonal: walks of one length
+  if (wgs <= 256) return steps >= 64 || (steps >= 16 && 5 * before <= 2 * (int64_t)p.Nk);
+  return wgs <= 512 && steps >= 32 && heads >= 6 && 10 * before <= p.Nk &&
+         4 * queries_after(p) <= p.Nq;
+}
+
+// dQ from dS in workgroups of four waves (128 queries), two per CU, instead of
+// sixteen (512 queries), one per CU.  They share each K tile among fewer waves
+// but put more CUs to work: with both forms in one round of the chip 0.5-0.8
+// of the time (2,000 tokens, 16 heads 73 -> 42 us; 4,096 x 4,096, 16 heads
+// 185 -> 156), and up to 192 large workgroups where the diagonal makes their
+// walks unequal (0.8-0.85).  Past that the large form streams dS the faster
+// (4,096 tokens, 32 heads 1.05, without a diagonal 1.1-1.2), and so it does
+// where 128 queries are all there are, its sixteen waves loading K for one
+// (17 queries over 20,000 keys, 9 heads 1.3-1.4 the time with four).
+bool dqds_four_waves(const Problem& p, int64_t heads) {
+  if (p.Nq <= 128) return false;
+  return heads * ((p.Nq + 127) / 128) <= 512 ||
+         (heads * ((p.Nq + 511) / 512) <= 192 && 5 * keys_before(p) <= p.Nk);
+}
+
 }  // namespace
 
 hipError_t launch_dq128(const Problem& p, const void* q, const void* k, const void* v,
@@ -916,17 +963,7 @@ hipError_t launch_dkdv128(const Problem& p, const void* q, const void* k, const 
     a.ds_nkb = (p.Nk + kDsBlockKeys - 1) / kDsBlockKeys;
   }
   const int64_t heads = (int64_t)p.Hkv * p.B;
-  // Few workgroups leave the chip idle, and with a diagonal the longest walk
-  // sets the time: four groups then split each walk (4,096 tokens, 32/8 heads,
-  // causal: 615 -> 361 us; 2,000 tokens, 16 heads 89 -> 63; 500 tokens, 32/8
-  // heads 88 -> 41; 8,192 tokens, 32/8 heads, 512 workgroups: 1350 -> 1210).
-  // They share tiles among two waves instead of four, so a grid that fills the
-  // chip evenly keeps one group (4,096 tokens, 16 heads, no diagonal, 512
-  // workgroups: 262 us against 372; causal 8,192 tokens, 16 heads, 1024: 555
-  // against 578).
-  const int64_t wgs = heads * ((p.Nk + 127) / 128);
-  const bool diagonal = p.causal && p.k_pos0 + p.Nk - 1 > p.q_pos0;
-  if (wgs <= (diagonal ? 512 : 128)) {
+  if (split_walks(p, heads * ((p.Nk + 127) / 128), heads)) {
     a.n_tiles = (p.Nk + 63) / 64;
     hipLaunchKernelGGL((dkdv128_kernel<2, 4>), dim3(a.n_tiles * heads), dim3(512), 0, s, a);
   } else {
@@ -950,11 +987,7 @@ hipError_t launch_dqds128(const Problem& p, const void* k, const uint16_t* ds, i
   a.ds_nqt = ds_nqt;
   a.ds_nkb = ds_nkb;
   const int64_t heads = (int64_t)p.Hq * p.B;
-  // Workgroups of four waves, two per CU, where 512-query ones would be at most
-  // one per CU (2,000 tokens, 16 heads: 73 -> 42 us; 2,048 tokens, 9 heads
-  // 92 -> 45; 4,096 x 4,096 tokens, 16 heads 185 -> 156); larger grids stream
-  // dS the faster the more waves share each K tile.
-  if (heads * ((p.Nq + 511) / 512) <= 256) {
+  if (dqds_four_waves(p, heads)) {
     a.n_tiles = (p.Nq + 127) / 128;
     hipLaunchKernelGGL(dqds128_kernel<4>, dim3(a.n_tiles * heads), dim3(256), 0, s, a);
   } else {

@@ -1,6 +1,7 @@
 """The head_dim 128 backward in each of its forms: dK/dV with four 32-key
 waves per workgroup, or two key waves x four query splits (small grids), and dQ
-from stored dS in workgroups of sixteen or four waves; at tile edges, with and
+from stored dS in workgroups of sixteen waves (up to 128 queries, and large
+grids) or four; at tile edges, with and
 without a diagonal, full and partial dS workspaces, against the float64 dense
 oracle (bf16 bar 2e-2 norm-relative)."""
 
@@ -14,14 +15,19 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     # b, nq, nk, hq, hkv, q_pos0, k_pos0, causal, valid
-    # two key waves x four splits (at most 512 workgroups of 128 keys, 128 without a diagonal)
+    # two key waves x four splits: at most 128 workgroups of 128 keys ...
     (1, 1, 1, 1, 1, 0, 0, True, None),            # one step for four groups
     (1, 33, 65, 2, 1, 40, 0, True, None),         # two steps a head, ragged key block
     (1, 95, 64, 6, 2, 0, 0, True, 50),            # nine steps over a group of three
     (2, 160, 200, 4, 1, 0, 0, True, None),        # the diagonal inside the walk
     (1, 70, 129, 2, 2, 200, 0, True, 150),        # no diagonal, valid_length
     (1, 130, 90, 3, 3, 0, 60, True, None),        # queries before every key
-    # four key waves, one walk (and sixteen-wave dQ from 257 heads x 512 queries on)
+    # ... 256 with long walks or most keys on the diagonal, 512 with nearly all of them there
+    (1, 520, 560, 48, 48, 40, 0, True, None),     # 240 workgroups
+    (1, 700, 720, 90, 30, 20, 0, True, None),     # 180; four-wave dQ past 512 workgroups
+    (1, 1030, 1040, 40, 40, 10, 0, True, 1037),   # 360
+    # four key waves, one walk
+    (1, 140, 3000, 16, 8, 2860, 0, True, None),   # 192 workgroups, walks of a few steps
     (4, 97, 300, 64, 64, 150, 0, True, None),     # 768 workgroups, diagonal
     (3, 40, 200, 66, 22, 300, 0, True, 190),      # 132, no diagonal, group of three
     (5, 33, 70, 56, 56, 20, 0, False, None),      # non-causal, 280 heads
