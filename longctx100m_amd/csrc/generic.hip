@@ -163,19 +163,28 @@ __device__ __forceinline__ void load_cols(float (&x)[4][NJ], const T* base, int6
 __device__ __forceinline__ void phase() { __builtin_amdgcn_sched_barrier(0); }
 
 // S (or dP) of one 16 x 16 tile: rows of a against the stationary rows b.
-// Two accumulators halve the dependent chain.
-template <int NJ, typename Frag>
+// Two accumulators halve the dependent chain; PARTS restarts keep the sums as
+// short as four-lane dot products have them (two: the output of 1,000 causal
+// tokens, 32/8 heads of 128, is 2.8e-7 from float64, with one 3.1e-7).
+template <int NJ, int PARTS, typename Frag>
 __device__ __forceinline__ f32x4 score_tile(const f32x4 (&a)[NJ], const Frag& b) {
-  f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+  constexpr int kPer = NJ >= PARTS ? NJ / PARTS : NJ;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const f32x4 bj = b[j];
-    s0 = mfma16x16x4(a[j][0], bj[0], s0);
-    s1 = mfma16x16x4(a[j][1], bj[1], s1);
-    s0 = mfma16x16x4(a[j][2], bj[2], s0);
-    s1 = mfma16x16x4(a[j][3], bj[3], s1);
+  for (int j0 = 0; j0 < NJ; j0 += kPer) {
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+    for (int j = j0; j < j0 + kPer; ++j) {
+      const f32x4 bj = b[j];
+      s0 = mfma16x16x4(a[j][0], bj[0], s0);
+      s1 = mfma16x16x4(a[j][1], bj[1], s1);
+      s0 = mfma16x16x4(a[j][2], bj[2], s0);
+      s1 = mfma16x16x4(a[j][3], bj[3], s1);
+    }
+    sum = j0 == 0 ? s0 + s1 : sum + (s0 + s1);
+    if (j0 + kPer < NJ) phase();  // one part's registers at a time
   }
-  return s0 + s1;
+  return sum;
 }
 
 // Stationary row fragments: in registers, or (kLds) in LDS, one copy for the
@@ -280,7 +289,10 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void fwd_generic_kernel(GenArgs
   for (int t = ksub; t < ntiles; t += a.split) {
     f32x4 s[NB];
 #pragma unroll
-    for (int n = 0; n < NB; ++n) s[n] = score_tile<NJ>(kr, qr[n]);
+    for (int n = 0; n < NB; ++n) {
+      s[n] = score_tile<NJ, 2>(kr, qr[n]);
+      phase();
+    }
     const bool more = t + a.split < ntiles;
     phase();
     if (more) load_rows<T, NJ>(kr, kb, ks, 16 * (t + a.split), a.Nk, D, vec, c, g);
@@ -303,11 +315,8 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void fwd_generic_kernel(GenArgs
       }
       const float muse = mnew == -INFINITY ? 0.f : mnew;  // no key yet: p = 0
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float p = expf(s[n][i] - muse);
-        l[n] += p;
-        s[n][i] = p;
-      }
+      for (int i = 0; i < 4; ++i) s[n][i] = expf(s[n][i] - muse);
+      l[n] += (s[n][0] + s[n][1]) + (s[n][2] + s[n][3]);
     }
 #pragma unroll
     for (int n = 0; n < NB; ++n) accumulate_tile<NJ>(o[n], vc, s[n]);
@@ -432,11 +441,11 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dq_generic_kernel(GenArgs 
   }
   for (int t = ksub; t < ntiles; t += a.split) {
     const bool more = t + a.split < ntiles;
-    const f32x4 s = score_tile<NJ>(kr, qr);
+    const f32x4 s = score_tile<NJ, 2>(kr, qr);
     phase();
     float kc[4][NJ];
     load_cols<T, NJ>(kc, kb, ks, 16 * t, a.Nk, D, vec, c, g);
-    const f32x4 dp = score_tile<NJ>(vr, dor);
+    const f32x4 dp = score_tile<NJ, 2>(vr, dor);
     phase();
     if (more) load_rows<T, NJ>(kr, kb, ks, 16 * (t + a.split), a.Nk, D, vec, c, g);
     f32x4 ds;
@@ -571,11 +580,11 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dkdv_generic_kernel(GenArg
       lse[i] = ok ? a.lse2[si + row] : INFINITY;
       dl[i] = ok ? a.delta[si + row] : 0.f;
     }
-    const f32x4 s = score_tile<NJ>(qr, kr);
+    const f32x4 s = score_tile<NJ, NJ <= 4 ? 2 : 1>(qr, kr);
     phase();
     float oc[4][NJ], qc[4][NJ];
     load_cols<T, NJ>(oc, obase(step), qs, qrow0, a.Nq, D, vec, c, g);
-    const f32x4 dp = score_tile<NJ>(dor, vr);
+    const f32x4 dp = score_tile<NJ, NJ <= 4 ? 2 : 1>(dor, vr);
     phase();
     load_cols<T, NJ>(qc, qbase(step), qs, qrow0, a.Nq, D, vec, c, g);
     f32x4 p, ds;

@@ -74,3 +74,34 @@ def test_fp32_math_edges(gpu, case):
     for got, e in zip(acc, want):
         # the sum with the starting one rounds at one ulp of a number of the gradient's size plus one
         assert np.abs(got.cpu().numpy() - 1 - e).max() <= TOL * (1 + np.abs(e).max())
+
+
+def _fma(a, b, c):
+    """fp32 fused multiply-add: the product of two fp32 values is exact in float64."""
+    return (a.double() * b.double() + c.double()).float()
+
+
+@pytest.mark.parametrize("d", [64, 96, 128])
+def test_scores_as_exact_as_four_lane_dot_products(gpu, d):
+    """The rounding of the scores, seen in the row maxima: on average no larger
+    than that of plain fp32 dot products of four chains of d / 4 fused
+    multiply-adds.  (10%: three standard deviations of the mean of 2,000
+    errors; two chains of twice the length are 1.4 times as far off.)"""
+    from longctx100m_amd import ring_attention as ra
+
+    n, heads = 1000, 32
+    g = gpu.Generator().manual_seed(d)
+    q, k, v = (gpu.randn(2, n, h, d, generator=g) for h in (heads, 8, 8))
+    _, m, _ = ra.fwd_shard(*(x.cuda() for x in (q, k, v)), q_pos0=0, k_pos0=0, causal=False)
+    got = lim = 0.0
+    for h in (0, 31):
+        qh, kh = q[0, :, h], k[0, :, h // 4]
+        exact = (qh.double() @ kh.double().T * d ** -0.5).max(1).values
+        part = [gpu.zeros(n, n) for _ in range(4)]
+        for j in range(0, d, 4):
+            for e in range(4):
+                part[e] = _fma(qh[:, j + e, None], kh[None, :, j + e], part[e])
+        s = ((part[0] + part[1]) + (part[2] + part[3])) * gpu.tensor(d ** -0.5).float()
+        lim += float((s.max(1).values.double() - exact).abs().mean())
+        got += float((m[0, h].cpu().double() - exact).abs().mean())
+    assert got <= 1.1 * lim, (got, lim)
