@@ -192,22 +192,11 @@ __device__ __forceinline__ f32x4 sum_parts(const uint8_t* smem, int wave0, int s
   return acc;
 }
 
-// The thread's rows r0, r0 + 4 split, ... < min(kRows, nrows) of a summed partial block to
-// the gradient, four rows at a time (grad_add); at(r): element of row r.
-template <int W, typename At>
-__device__ __forceinline__ void grad_rows(float* dst, uint16_t* out, int init, int split, int r0,
-                                          int nrows, const At& at, const uint8_t* smem, int wave0,
-                                          int off) {
-  for (int base = r0; base < kRows; base += 16 * split) {
-    f32x4 v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = min(base + 4 * split * j, kRows - 1);
-      v[j] = sum_parts<W>(smem, wave0, split, r * kPitch + off);
-    }
-    grad_add(dst, out, init, v, [&](int j) { return at(base + 4 * split * j); },
-             [&](int j) { return base + 4 * split * j < min(kRows, nrows); });
-  }
+// What an accumulator holds before a contribution (init: nothing).
+__device__ __forceinline__ f32x4 grad_old(const float* acc, int init, int64_t i) {
+  f32x4 r = {0.f, 0.f, 0.f, 0.f};
+  if (!init) r = *reinterpret_cast<const f32x4*>(acc + i);
+  return r;
 }
 
 // ----------------------------------------------------------------- forward --
@@ -496,11 +485,15 @@ __global__ __launch_bounds__(64 * W, 2) void dq64_kernel(Args64 a) {
     if (n > 0) __syncthreads();
     store_part(reinterpret_cast<float*>(mem), acc[n], a.scale, lane);
     __syncthreads();
-    const int r0 = 4 * ksub + (lane >> 4), d = 4 * (lane & 15);
-    grad_rows<W>(
-        a.dq, a.out, a.init, a.split, r0, a.Nq - (q0 + kRows * n),
-        [&](int r) { return (((int64_t)b * a.Nq + q0 + kRows * n + r) * a.Hq + h) * D + d; },
-        smem, qsub * a.split, d);
+    for (int r = 4 * ksub + (lane >> 4); r < kRows; r += 4 * a.split) {
+      const int row = q0 + kRows * n + r;
+      if (row >= a.Nq) break;
+      const int d = 4 * (lane & 15);
+      const int64_t i = (((int64_t)b * a.Nq + row) * a.Hq + h) * D + d;
+      const f32x4 old = grad_old(a.dq, a.init, i);  // on its way during the sum
+      store4(a.dq + i, a.out != nullptr ? a.out + i : nullptr,
+             old + sum_parts<W>(smem, qsub * a.split, a.split, r * kPitch + d));
+    }
   }
 }
 
@@ -642,10 +635,16 @@ __global__ __launch_bounds__(64 * W, 2) void dkdv64_kernel(Args64 a) {
   store_part(reinterpret_cast<float*>(mem), dk, a.scale, lane);
   store_part(reinterpret_cast<float*>(mem) + kPart, dv, 1.f, lane);
   __syncthreads();
-  const int r0 = 4 * qsub + (lane >> 4), d = 4 * (lane & 15);
-  auto at = [&](int r) { return (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D + d; };
-  grad_rows<W>(a.dk, a.dk16, a.init, a.split, r0, a.Nk - k0, at, smem, ksub * a.split, d);
-  grad_rows<W>(a.dv, a.dv16, a.init, a.split, r0, a.Nk - k0, at, smem, ksub * a.split, kPart + d);
+  for (int r = 4 * qsub + (lane >> 4); r < kRows; r += 4 * a.split) {
+    if (k0 + r >= a.Nk) break;
+    const int d = 4 * (lane & 15);
+    const int64_t i = (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D + d;
+    const f32x4 oldk = grad_old(a.dk, a.init, i), oldv = grad_old(a.dv, a.init, i);
+    store4(a.dk + i, a.dk16 != nullptr ? a.dk16 + i : nullptr,
+           oldk + sum_parts<W>(smem, ksub * a.split, a.split, r * kPitch + d));
+    store4(a.dv + i, a.dv16 != nullptr ? a.dv16 + i : nullptr,
+           oldv + sum_parts<W>(smem, ksub * a.split, a.split, kPart + r * kPitch + d));
+  }
 }
 
 Args64 make_args(const Problem& p, const void* q, const void* k, const void* v, const void* dout) {
