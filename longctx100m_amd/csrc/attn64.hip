@@ -54,7 +54,6 @@ constexpr int kPitch = D + 4;             // floats per row of a wave's partial
 constexpr int kPart = kRows * kPitch;     // floats of a partial block
 // A wave's LDS: two buffers of two tiles, later its partial(s).
 constexpr int kWaveLds = 4 * kTile > 2 * kPart * 4 ? 4 * kTile : 2 * kPart * 4;
-constexpr float kRescaleSlack = 8.0f;     // log2 units
 
 struct Args64 {
   const uint16_t* q;
@@ -206,7 +205,7 @@ __device__ __forceinline__ f32x4 grad_old(const float* acc, int init, int64_t i)
 template <int NQ, int W>
 __global__ __launch_bounds__(64 * W, 2) void fwd64_kernel(Args64 a) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[W * kWaveLds];
-  __shared__ float rsm[W][kRows], tsm[W][kRows], lsm[W][kRows], rtop[W][kRows], ttop[W][kRows];
+  __shared__ float msm[W][kRows], lsm[W][kRows], mtop[W][kRows];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 31, hh = lane >> 5;
@@ -241,13 +240,13 @@ __global__ __launch_bounds__(64 * W, 2) void fwd64_kernel(Args64 a) {
 
   bf16x8 qr[NQ][4];
   f32x16 o[NQ][2];
-  float mrun[NQ], mtrue[NQ], lsum[NQ];  // reference and exact maximum (log2 units), partial sum
+  float mrun[NQ], lsum[NQ];  // running maximum (log2 units), partial sum
   int klim[NQ];
 #pragma unroll
   for (int n = 0; n < NQ; ++n) {
     load_stationary(qr[n], qb, qs, q0 + kRows * n, a.Nq, lane);
     o[n][0] = o[n][1] = f32x16{};
-    mrun[n] = mtrue[n] = -INFINITY;
+    mrun[n] = -INFINITY;
     lsum[n] = 0.f;
     klim[n] = visible_keys(a, min(q0 + kRows * n + c, a.Nq - 1));
   }
@@ -272,23 +271,23 @@ __global__ __launch_bounds__(64 * W, 2) void fwd64_kernel(Args64 a) {
 #pragma unroll
       for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[n][v]);
       mx = xor32_max(mx) * a.sl2;
-      mtrue[n] = fmaxf(mtrue[n], mx);
-      const bool raise = mx > mrun[n] + kRescaleSlack;
-      if (__any(raise)) {
-        const float mnew = raise ? mx : mrun[n];
-        const float alpha = raise ? fast_exp2(mrun[n] - mnew) : 1.f;  // mrun = -inf: 0
+      if (__any(mx > mrun[n])) {
+        const float mnew = fmaxf(mrun[n], mx);
+        const float alpha = mx > mrun[n] ? fast_exp2(mrun[n] - mnew) : 1.f;  // mrun = -inf: 0
         mrun[n] = mnew;
         lsum[n] *= alpha;
         o[n][0] *= alpha;
         o[n][1] *= alpha;
       }
       const float muse = mrun[n] == -INFINITY ? 0.f : mrun[n];  // no key yet: p = 0
+      float ts = 0.f;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const float p = fast_exp2(fmaf(s[n][v], a.sl2, -muse));
-        lsum[n] += p;
+        ts += p;
         s[n][v] = p;
       }
+      lsum[n] += ts;
       pb[n][0] = pack_scores(s[n], 0);
       pb[n][1] = pack_scores(s[n], 1);
       phase();
@@ -310,33 +309,25 @@ __global__ __launch_bounds__(64 * W, 2) void fwd64_kernel(Args64 a) {
     tile(kt, kt + kTile, t * kRows);
   }
 
-  // The key splits of each query merge by log-sum-exp (o and l relative to the
-  // reference maximum, l converted to the exact one); accumulate: then into
+  // The key splits of each query merge by log-sum-exp; accumulate: then into
   // the running state of the row with lc_attn_merge's weights.
   const int p0 = qsub * a.split;
 #pragma unroll
   for (int n = 0; n < NQ; ++n) {
     const float ln = xor32_sum(lsum[n]);
-    float R = mrun[n], T = mtrue[n];
+    float M = mrun[n];
     if (n > 0) __syncthreads();
     if (a.split > 1) {
-      if (hh == 0) {
-        rsm[wave][c] = R;
-        tsm[wave][c] = T;
-      }
+      if (hh == 0) msm[wave][c] = M;
       __syncthreads();
 #pragma unroll
-      for (int s = 0; s < W; ++s) {
-        R = fmaxf(R, rsm[p0 + min(s, a.split - 1)][c]);
-        T = fmaxf(T, tsm[p0 + min(s, a.split - 1)][c]);
-      }
+      for (int s = 0; s < W; ++s) M = fmaxf(M, msm[p0 + min(s, a.split - 1)][c]);
     }
-    const float f = mrun[n] == -INFINITY ? 0.f : fast_exp2(mrun[n] - R);  // 1 without splits
+    const float f = mrun[n] == -INFINITY ? 0.f : fast_exp2(mrun[n] - M);  // 1 without splits
     store_part(reinterpret_cast<float*>(mem), o[n], f, lane);
     if (hh == 0) {
       lsm[wave][c] = ln * f;
-      rtop[wave][c] = R;
-      ttop[wave][c] = T;
+      mtop[wave][c] = M;
     }
     __syncthreads();
     // 16 threads per row; the waves of the query block take its rows in turn.
@@ -351,15 +342,14 @@ __global__ __launch_bounds__(64 * W, 2) void fwd64_kernel(Args64 a) {
         const float x = lsm[p0 + min(s, a.split - 1)][r];
         lt += s < a.split ? x : 0.f;
       }
-      const float top = ttop[p0][r];
+      const float top = mtop[p0][r];
       const float inv = lt > 0.f ? 1.f / lt : 0.f;
-      const float ltrue = lt > 0.f ? lt * fast_exp2(rtop[p0][r] - top) : 0.f;
       const float mnat = top == -INFINITY ? -INFINITY : top * kLn2;
       const int64_t si = ((int64_t)b * a.Hq + h) * a.Nq + row;
       const int64_t oi = (((int64_t)b * a.Nq + row) * a.Hq + h) * D + d;
       uint16_t* out = a.out != nullptr ? a.out + oi : nullptr;
       if (a.accumulate) {
-        const MergeW w = merge_weights(a.m[si], a.l[si], mnat, ltrue);
+        const MergeW w = merge_weights(a.m[si], a.l[si], mnat, lt);
         store4(a.o + oi, out, *reinterpret_cast<const f32x4*>(a.o + oi) * w.wa + acc * (w.wb * inv));
         // every thread of the row has read the old statistics: they are in one wave
         if (d == 0) {
@@ -370,7 +360,7 @@ __global__ __launch_bounds__(64 * W, 2) void fwd64_kernel(Args64 a) {
         store4(a.o + oi, out, acc * inv);
         if (d == 0) {
           a.m[si] = mnat;
-          a.l[si] = ltrue;
+          a.l[si] = lt;
         }
       }
     }
