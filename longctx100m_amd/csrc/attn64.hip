@@ -712,8 +712,16 @@ int fwd_split(int64_t blocks, int64_t tiles, int over, int keep) {
   return s;
 }
 
-// Blocks of 64 stationary rows per wave once those fill the chip.
-bool two_blocks(int64_t blocks) { return blocks >= 2 * kWaveSlots; }
+// Blocks of 64 stationary rows per wave once those fill the chip, given rows
+// for the second half.
+bool two_blocks(int64_t blocks, int rows) { return blocks >= 2 * kWaveSlots && rows > kRows; }
+
+// Splits for which a workgroup's four waves all have rows: a head with one or
+// two row blocks has the others take keys (16 queries over 500 keys, 128 x 32/8
+// heads: 109 us with three waves idle, 52 with all four on the keys).
+int least_split(int rows, int per_wave) {
+  return rows <= per_wave ? 4 : rows <= 2 * per_wave ? 2 : 1;
+}
 
 }  // namespace
 
@@ -730,9 +738,10 @@ hipError_t launch_fwd64(const Problem& p, const void* q, const void* k, const vo
   a.m = m;
   a.l = l;
   const int64_t heads = (int64_t)p.B * p.Hq, blocks = heads * ((p.Nq + kRows - 1) / kRows);
-  const bool two = two_blocks(blocks);
+  const bool two = two_blocks(blocks, p.Nq);
   const int64_t tiles = (p.Nk + kRows - 1) / kRows;
   a.split = two ? std::min(4, fwd_split(blocks / 2, tiles, 4, 32)) : fwd_split(blocks, tiles, 2, 16);
+  a.split = std::max(a.split, least_split(p.Nq, two ? 2 * kRows : kRows));
   const int nw = a.split == 8 ? 8 : 4, rows = nw / a.split * kRows * (two ? 2 : 1);
   a.n_tiles = (p.Nq + rows - 1) / rows;
   const dim3 grid((unsigned)(a.n_tiles * heads));
@@ -753,9 +762,10 @@ hipError_t launch_dq64(const Problem& p, const void* q, const void* k, const voi
   a.delta = delta;
   a.dq = dq;
   const int64_t heads = (int64_t)p.B * p.Hq, blocks = heads * ((p.Nq + kRows - 1) / kRows);
-  const bool two = two_blocks(blocks);
+  const bool two = two_blocks(blocks, p.Nq);
   const int64_t tiles = (p.Nk + kRows - 1) / kRows;
   a.split = two ? std::min(4, split_for(blocks / 2, tiles, 4)) : split_for(blocks, tiles, 2);
+  a.split = std::max(a.split, least_split(p.Nq, two ? 2 * kRows : kRows));
   const int nw = a.split == 8 ? 8 : 4, rows = nw / a.split * kRows * (two ? 2 : 1);
   a.n_tiles = (p.Nq + rows - 1) / rows;
   const dim3 grid((unsigned)(a.n_tiles * heads));

@@ -22,6 +22,9 @@ CASES = [
     (1, 70, 90, 2, 1, 0, 0, False, None),          # non-causal
     (1, 64, 1024, 9, 3, 960, 0, True, None),       # eight key splits
     (1, 1000, 64, 6, 1, 0, 0, True, 50),           # dK/dV: eight splits over a group of six
+    (64, 20, 70, 64, 16, 50, 0, True, None),       # one row block per head: four waves on its keys
+    (32, 50, 70, 64, 16, 20, 0, True, 65),         # two (64-row waves for 2,048 heads): ragged
+    (8, 100, 64, 16, 16, 0, 0, False, None),       # more waves than tiles
     (2, 2100, 300, 40, 20, 100, 0, True, None),    # 64-row waves with key splits
     (1, 1100, 2200, 128, 128, 1100, 0, True, 2150),  # 64-row waves, ragged tail block
 ]
