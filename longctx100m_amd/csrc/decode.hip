@@ -526,8 +526,11 @@ int waves_for(const Problem& p) {
 // wave would walk twelve tiles eight per CU even out the CUs' rates (64 KV
 // heads x 50,000 keys of 64 135 us against 150 with four, 256 heads x 60,000
 // 1.22 ms against 1.33); short caches take a tile per wave (4,000 keys 9.8 us
-// against 11.6 at two), and up to four tiles a wave one workgroup is as fast as
-// the merge it saves (500 keys: 7.8 us against 7.6; 300 keys 6.4 against 8.1).
+// against 11.6 at two).  Up to four tiles a wave one workgroup saves the merge's
+// launch: on the GPU it is as fast to 300 keys of 128 and slower from there (512
+// keys, 8 KV heads 12.2 us against 8.6, one CU reading what four could), but a
+// call from Python takes 14.7 us against 17.6, and a decoder layer, bound by
+// the GPU, 88.8 against 87.1 at 500 keys and 86.0 against 87.5 at 300.
 int choose_splits(const Problem& p) {
   const int64_t units = (int64_t)p.B * p.Hkv * row_blocks(p);
   const int tk = kTileBytes / (2 * p.D);
@@ -566,6 +569,28 @@ int64_t fixed_splits(const Problem& p) {
   return std::min<int64_t>(std::min<int64_t>(std::max<int64_t>(1, want), most), 4096);
 }
 
+// Where the blockwise forward (one walk of the cache per query head, up to 128
+// query rows at once) is not the better choice; the shapes with a required
+// workspace run here in any case.  Times are this kernel's over the forward's.
+bool splits_pay(const Problem& p) {
+  const int64_t rb = row_blocks(p), units = (int64_t)p.B * p.Hkv * rb, group = p.Hq / p.Hkv;
+  const int64_t tk = kTileBytes / (2 * p.D), tiles = ((int64_t)p.Nk + tk - 1) / tk;
+  // A full chip of heads that share KV heads: the forward walks each cache
+  // `group` times (64 sequences, 32/8 heads, 8 tokens: 0.4-0.9).
+  if (group >= 4 * rb && (int64_t)p.B * p.Hq > 256) return true;
+  // Otherwise long caches of few sequences.  head_dim 128: the forward is as
+  // fast on the first few hundred keys (1.0-1.2) and, reading the cache once
+  // for all rows, on grids of 256 and more (64 rows: 1.3-2.4, 17 rows over
+  // 2,000 keys and more 1.0-1.3).
+  if (p.D == 128) return units < 256 && tiles > 6 * (rb + 1);
+  // head_dim 64: the forward splits keys over its waves too, which is as good
+  // as one workgroup per unit (up to 1,024 keys 1.0-1.4, and 0.7-0.9 from 2,000
+  // on); with two row blocks it takes more keys per sequence (8 KV heads: 1.9
+  // at 1,000 keys, 0.9 at 2,000; 32: 1.0 at 4,000; 128 and more: 1.3-2.1).
+  if (rb == 1) return units < 512 && tiles > 16;
+  return units < 256 && tiles > std::max<int64_t>(24, units);
+}
+
 }  // namespace
 
 int decode_splits(const Problem& p) {
@@ -575,7 +600,7 @@ int decode_splits(const Problem& p) {
 
 bool decode_supported(const Problem& p) {
   return p.dtype == 1 && !p.precise && (p.D == 64 || p.D == 128) && p.Nq > 0 &&
-         (int64_t)p.Nq * (p.Hq / p.Hkv) <= kDecodeMaxRows;
+         (int64_t)p.Nq * (p.Hq / p.Hkv) <= kDecodeMaxRows && (fixed_workspace(p) || splits_pay(p));
 }
 
 bool decode_workspace_required(const Problem& p) { return fixed_workspace(p); }

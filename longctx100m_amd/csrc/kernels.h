@@ -119,7 +119,8 @@ hipError_t launch_bwd_preprocess(int B, int N, int H, int D, int dtype, const vo
                                  float* lse2, hipStream_t s);
 
 // Split-KV decode attention (decode.hip): bf16, D = 64 or 128, one to
-// kDecodeMaxRows query rows (Nq * Hq / Hkv) per KV head.
+// kDecodeMaxRows query rows (Nq * Hq / Hkv) per KV head, where it is faster than
+// the blockwise kernels (or its workspace is required).
 // decode_workspace_required: a workspace of decode_workspace_bytes must be
 // given (D = 128, at most 16 rows); other shapes may run the blockwise kernels
 // instead, and need none when decode_workspace_bytes is 0.

@@ -51,7 +51,8 @@ DECODE_CASES = [
     (1, 2, 4, 4, 1000, 0, 131072, True, 131072 + 777),  # offset cache, valid_length cut
     (1, 3, 8, 8, 4096, -40, 0, True, None),       # queries inside the cache (causal masks keys)
     (1, 1, 8, 8, 64, 0, 0, False, None),          # tiny cache, non-causal
-    (1, 8, 8, 2, 2000, 0, 0, True, None),         # 32 rows: the blockwise fallback
+    (1, 8, 8, 2, 2000, 0, 0, True, None),         # 32 rows: the split kernel, two row halves
+    (1, 13, 10, 2, 2000, 0, 0, True, None),       # 65 rows: the blockwise kernels
 ]
 
 
@@ -73,9 +74,9 @@ def test_decode_matches_dense(ra, gpu, case):
 
 def _random_decode_cases(seed, n):
     """Random decode geometries (drawn once), in DECODE_CASES' tuple form: batch,
-    1-4 new tokens, GQA groups up to 8 (16 or fewer rows per KV head take the
-    split kernel, more the blockwise fallback), caches of 1 to 20,000 keys at
-    an offset, queries anywhere from before the first key to the cache end,
+    1-4 new tokens, GQA groups up to 8 (16 or fewer rows per KV head always take
+    the split kernel, 17 to 32 from a few hundred keys on), caches of 1 to 20,000
+    keys at an offset, queries anywhere from before the first key to the cache end,
     causal or not, valid_length inside or past the cache."""
     rng = np.random.default_rng(seed)
     out = []

@@ -139,3 +139,30 @@ def test_split_workspace_sizes():
     for nq in (1, 100, 500, 2000):
         for hq in (1, 9, 32, 500):
             assert _bytes(lib, sh(1, nq, 65536, hq, 1, 128, bf)) <= 36 << 20
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,accumulate", [(128, False), (128, True), (64, False)])
+def test_infinite_value_reaches_its_column_alone(gpu, d, accumulate):
+    """An infinity in one value that every query sees: that dim of the KV head's
+    rows is infinite after the merge of the splits (head_dim 64: of the waves),
+    also into a running state, and the others are what they were."""
+    from longctx100m_amd import ring_attention as ra
+
+    nq, nk = 40, 3000
+    rng = np.random.default_rng(d)
+    q, k, v = (bf16_round(rng.standard_normal(s, dtype=np.float32))
+               for s in ((1, nq, 4, d), (1, nk, 2, d), (1, nk, 2, d)))
+    qt, kt, vt = (gpu.tensor(x).to(gpu.bfloat16).cuda() for x in (q, k, v))
+    kw = dict(q_pos0=0, k_pos0=0, causal=False)
+    eo, _, _ = dense.attention_fwd(q, k, v, **kw)
+    state = {}
+    if accumulate:  # the same hop before: the merge keeps o
+        state = dict(zip("oml", ra.fwd_shard(qt, kt, vt, **kw)))
+    vt[0, 1234, 1, 7] = float("inf")
+    o, _, _ = ra.fwd_shard(qt, kt, vt, **kw, **state, accumulate=accumulate)
+    got = o.cpu().numpy()
+    hit = np.zeros(got.shape, bool)
+    hit[0, :, 2:, 7] = True
+    assert np.all(got[hit] == np.inf)
+    assert norm_rel(got[~hit], eo[~hit]) <= 2e-2
