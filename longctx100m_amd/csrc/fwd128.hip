@@ -441,13 +441,16 @@ size_t split_bytes(const Problem& p, int S) {
 // Splits of workgroups of `waves` waves, of at least 512 keys each: what the
 // chip holds at two waves per SIMD (512 queries, 32/8 heads over 32,512 keys:
 // 555 us in 128 workgroups of four waves, 281 in 512 and their merge; 17
-// queries over 20,017 keys 329 us and 35; 1,000 over 11,000 246 and 200), or,
-// where the keys do not suffice for most of that, one workgroup per CU (100
-// queries over 5,100 keys: 26.7 us in 256 against 32.6 in 288).
+// queries over 20,017 keys 329 us and 35; 1,000 over 11,000 246 and 200), or
+// one workgroup per CU where the keys do not suffice for more: over 5,449
+// random shapes 257 to 399 workgroups take 1.02-1.12 of the time of up to 256
+// below 2,048 keys each and 0.72-0.98 from there on, 400 to 512 1.0-1.17 below
+// 1,024 and 0.7-0.9 from there on (100 queries over 5,100 keys: 26.7 us in 256,
+// 32.6 in 288; 1,000 over 2,047, 32/8 heads: 44 us in 256, i.e. unsplit, 50 in 512).
 static int splits_of(const Problem& p, int64_t waves) {
   const int64_t wgs = (p.Nq + waves * kQW - 1) / (waves * kQW) * p.Hq * p.B;
   int64_t s = std::min<int64_t>({256 * 8 / waves / wgs, p.Nk / kFwdSplitKeys, kFwdMaxSplits});
-  if (s * wgs > 256 && s * wgs < 400) s = 256 / wgs;
+  if (s * wgs > 256 && p.Nk < s * (s * wgs < 400 ? 2048 : 1024)) s = 256 / wgs;
   return (int)std::max<int64_t>(1, s);
 }
 
