@@ -96,9 +96,17 @@ int lc_attn_fwd_shard(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, 
  * tokens against many keys) has its keys split over more of them, and a second
  * kernel merges the splits by log-sum-exp.  Applies to d = 128 on the bf16 MFMA
  * path with up to 65,536 keys; lc_attn_fwd_shard_workspace_bytes returns the
- * bytes it needs (at most 36 MB), 0 for shapes that do not split.  With a smaller or misaligned
- * (16 bytes) workspace, or other shapes, this is lc_attn_fwd_shard.  Results
- * agree up to fp32 summation order. */
+ * bytes it needs (at most 36 MB), 0 for shapes that do not split.  With a
+ * smaller or misaligned (16 bytes) workspace, or other shapes, this is
+ * lc_attn_fwd_shard.
+ * Against the unsplit call m is the same, l agrees up to fp32 summation order
+ * (tested to 1e-5 norm-relative), and o up to the rounding of the probabilities
+ * to bf16, which each split does relative to its own maximum (about 2e-3
+ * norm-relative, tested to 1e-2; both are as far from the exact result).  The
+ * number of splits depends on the whole shape, batch included: a sequence's o
+ * can differ by that much between batches of another size.  The same holds for
+ * lc_attn_decode, lc_attn_decode_static and, given the workspace to split its
+ * hops, lc_ring_fwd_with_stats. */
 size_t lc_attn_fwd_shard_workspace_bytes(const lc_attn_shape_t* shape);
 int lc_attn_fwd_shard_ws(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, const void* q,
                          const void* k, const void* v, float* o, float* m, float* l,
@@ -113,8 +121,11 @@ int lc_attn_fwd_shard_ws(const lc_attn_shape_t* shape, const lc_attn_mask_t* mas
  * 16-byte-aligned workspace of lc_attn_decode_workspace_bytes(shape) bytes
  * (LC_ERR_WORKSPACE if smaller, LC_ERR_INVALID if misaligned); the other of
  * these shapes run the lc_attn_fwd_shard kernels when the workspace is
- * smaller or misaligned, and so do all further shapes (the size query returns
- * 0 where no workspace is used).
+ * smaller or misaligned or where those are the faster, and so do all further
+ * shapes (the size query returns 0 where no workspace is used).  A workspace
+ * of the query's size or more is written, so calls that share one must be
+ * ordered; before ABI version 3 head_dim 64 and more than 16 rows left it
+ * untouched.
  * No counterpart in the reference, whose generation loops recompute the whole
  * prefill for every new token (src/longctx100m/distributed_infer.py:185-219,
  * rust/longctx100m-model/src/bin/infer.rs:96-106); callers that keep a KV cache
@@ -134,7 +145,8 @@ int lc_attn_decode(const lc_attn_shape_t* shape, const lc_attn_mask_t* mask, con
  * rejected with LC_ERR_WORKSPACE (use lc_attn_decode); those that only may use
  * one run the lc_attn_fwd_shard kernels then.  Every call on one GPU shares its
  * array, so calls that overlap on one GPU (concurrent streams or threads)
- * race; calls ordered on a stream do not.  The array used is that of the
+ * race; calls ordered on a stream do not.  (Before ABI version 3 head_dim 64
+ * and more than 16 rows per KV head did not use the array.)  The array used is that of the
  * stream's device (the current device for a null stream).  Results equal
  * lc_attn_decode's. */
 #define LC_DECODE_STATIC_SCRATCH_BYTES ((size_t)16 << 20)
@@ -283,6 +295,13 @@ int lc_reference_causal_attention_host(int32_t batch, int32_t tokens, int32_t he
 /* ---- misc ------------------------------------------------------------------- */
 
 const char* lc_last_error(void);
+/* 3.  Version 3: lc_attn_decode writes a large enough workspace, and
+ * lc_attn_decode_static its array, for head_dim 64 and for 17 to 64 query rows
+ * per KV head too, which version 2 left untouched; lc_ring_fwd_with_stats
+ * writes workspace past its running output, up to the size query's bytes;
+ * lc_attn_fwd_shard_ws and its size query are new.  A caller of version 2 that
+ * shares such a buffer between overlapping calls, or passes one that is in
+ * other use, has to separate them. */
 int32_t lc_abi_version(void);
 
 #ifdef __cplusplus

@@ -368,7 +368,7 @@ extern "C" {
 
 const char* lc_last_error(void) { return g_last_error.c_str(); }
 
-int32_t lc_abi_version(void) { return 2; }
+int32_t lc_abi_version(void) { return 3; }
 
 size_t lc_attn_fwd_shard_workspace_bytes(const lc_attn_shape_t* shape) {
   if (check_shape(shape) != LC_OK) return 0;

@@ -132,7 +132,9 @@ def decode(q, k, v, *, q_pos0: int, k_pos0: int = 0, causal: bool = True,
            m: Optional[torch.Tensor] = None, l: Optional[torch.Tensor] = None,
            workspace: Optional[torch.Tensor] = None):
     """Split-KV decode of a few query tokens against a long KV shard (a KV
-    cache): same outputs as fwd_shard, (o [B,Nq,Hq,D] fp32, m, l [B,Hq,Nq])."""
+    cache): same outputs as fwd_shard, (o [B,Nq,Hq,D] fp32, m, l [B,Hq,Nq]).
+    A ``workspace`` that is large enough is written, so calls that overlap need
+    one each; without one a tensor of the current stream is allocated."""
     _check_dev(q, k, v)
     s = _shape(q, k, False)
     mk = _lib.Mask(q_pos0, k_pos0, _opt(valid_length), int(causal), 0)

@@ -78,7 +78,7 @@ static lc_ring_desc_t desc(int world, int rank, int n, int hq, int hkv, int d) {
 }
 
 static int validate(void) {
-  check(lc_abi_version() == 2, "lc_abi_version() == 2");
+  check(lc_abi_version() == 3, "lc_abi_version() == 3");
   float x = 0.f;
   const void* p[2] = {&x, &x};
   float* fp = &x;

@@ -34,7 +34,7 @@ def test_library_exports_every_declared_symbol(lib):
     assert sorted(_lib.SIGNATURES) == declared
     for name in declared:
         assert hasattr(lib, name), name
-    assert lib.lc_abi_version() == 2
+    assert lib.lc_abi_version() == 3
 
 
 def test_struct_layouts_match_header():
