@@ -122,11 +122,14 @@ __device__ __forceinline__ float group4_sum(float x) { return xor16_sum(xor32_su
 // l = e^{m_a-m} l_a + e^{m_b-m} l_b and o = (e^{m_a-m} l_a o_a + e^{m_b-m} l_b o_b) / l,
 // which equals carrying the reference's unnormalised (m, l, acc) across the
 // two partials (rs:36-53 applied blockwise).  No key seen on either side:
-// weights 0, l = 0, m = -inf.
+// weights 0, l = 0, m = -inf.  Nothing here is contracted into fused
+// multiply-adds, so that a merge in a kernel's epilogue and lc_attn_merge on the
+// stored partial give the same m and l, however the compiler arranges either.
 struct MergeW {
   float wa, wb, m, l;
 };
 __device__ __forceinline__ MergeW merge_weights(float ma, float la, float mb, float lb) {
+#pragma clang fp contract(off)
   MergeW w;
   w.m = fmaxf(ma, mb);
   if (w.m == -INFINITY) {
