@@ -53,8 +53,8 @@ EXTRA_FLAGS = {
 
 # Kernel (mangled-name substring) -> allowed scratch bytes per lane.  The
 # dK/dV kernel keeps a few loop-invariant mask values in scratch, reloaded only
-# on tiles that need the mask; at head_dim 128 the fp32-math forward and dQ keep
-# a few values of their prologue there, most of them until after the walk.
+# on tiles that need the mask; from head_dim 65 on the fp32-math kernels keep a
+# few values of their prologue there, most of them until after the walk.
 SCRATCH_LIMITS = {
     "fwd64_kernel": 0,
     "dq64_kernel": 0,
@@ -65,7 +65,7 @@ SCRATCH_LIMITS = {
     "dqds128_kernel": 0,
     "decode_kernel": 0,
     "rmsnorm_kernel": 0,
-    "generic_kernel": 20,
+    "generic_kernel": 24,
 }
 
 # "Function Name: <kernel>" starts a kernel's block; then "<field> [unit]: value".

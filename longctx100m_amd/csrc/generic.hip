@@ -580,7 +580,7 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dkdv_generic_kernel(GenArg
       lse[i] = ok ? a.lse2[si + row] : INFINITY;
       dl[i] = ok ? a.delta[si + row] : 0.f;
     }
-    const f32x4 s = score_tile<NJ, NJ <= 4 ? 2 : 1>(qr, kr);
+    const f32x4 s = score_tile<NJ, 2>(qr, kr);
     phase();
     float oc[4][NJ], qc[4][NJ];
     load_cols<T, NJ>(oc, obase(step), qs, qrow0, a.Nq, D, vec, c, g);
