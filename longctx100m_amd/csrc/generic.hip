@@ -605,31 +605,19 @@ __global__ __launch_bounds__(64 * max_waves(NJ)) void dkdv_generic_kernel(GenArg
   auto reduce = [&](const f32x4 (&acc)[NJ], float* dst, uint16_t* out, float scale) {
     store_part<NJ>(smem + wave * kPart, acc, c, g);
     __syncthreads();
-    // The wave's rows wave, wave + nw, ... (four with four waves, two with
-    // eight); the old values of all of them are read before the first sum.
-    for (int d = lane; d < D; d += 64) {
-      float old[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = wave + i * nw;
-        old[i] = 0.f;
-        if (!a.init && r < 16 && k0 + r < a.Nk)
-          old[i] = dst[(((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D + d];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = wave + i * nw;
-        if (r >= 16 || k0 + r >= a.Nk) break;
+    for (int r = wave; r < 16 && k0 + r < a.Nk; r += nw) {
+      const int64_t ki = (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D;
+      for (int d = lane; d < D; d += 64) {
+        const float old = a.init ? 0.f : dst[ki + d];  // on its way during the sum
         float sum = 0.f;
 #pragma unroll
         for (int w = 0; w < max_waves(NJ); ++w) {
           const float x = smem[min(w, nw - 1) * kPart + r * part_pitch(DP) + d];
           sum += w < nw ? x : 0.f;
         }
-        const int64_t ki = (((int64_t)b * a.Nk + k0 + r) * a.Hkv + hk) * D + d;
-        const float x = old[i] + sum * scale;
-        if (out != nullptr) out[ki] = f32_to_bf16(x);
-        else dst[ki] = x;
+        const float x = old + sum * scale;
+        if (out != nullptr) out[ki + d] = f32_to_bf16(x);
+        else dst[ki + d] = x;
       }
     }
   };
