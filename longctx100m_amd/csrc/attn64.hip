@@ -34,10 +34,10 @@
 // in the forward, 384 in dQ, 512 in dK/dV) and the softmax's VALU work (about
 // 450) hardly overlap; waits for the DMA are 2-8% of the walk.  Measured,
 // causal, against workgroups of four 32-row waves sharing register-staged
-// tiles, 16x16x32 MFMA: 2 x 2,047 tokens, 9/3 heads, forward 73 -> 41 us, dQ
-// 112 -> 41, dK/dV 424 -> 45; 4,096 tokens, 32/8 heads 185 -> 130, 385 -> 150,
-// 1117 -> 195; 16,384 tokens, 16 heads 1.00 -> 0.80 ms (690 TFLOP/s), 2.52 ->
-// 0.90 (917), 4.62 -> 1.30 (848).
+// tiles, 16x16x32 MFMA (GPU time of a call): 2 x 2,047 tokens, 9/3 heads, forward
+// 66 -> 36 us, dQ 105 -> 39, dK/dV 421 -> 42; 4,096 tokens, 32/8 heads 167 -> 120,
+// 365 -> 141, 1130 -> 191; 16,384 tokens, 16 heads 0.89 -> 0.72 ms (770 TFLOP/s),
+// 2.60 -> 0.90 (917), 4.65 -> 1.30 (848).
 #include "common.h"
 #include "kernels.h"
 #include "tile128.h"
@@ -679,15 +679,13 @@ Args64 make_args(const Problem& p, const void* q, const void* k, const void* v, 
 
 constexpr int64_t kWaveSlots = 2048;  // waves the chip holds (two per SIMD)
 
-// Waves that share a block of stationary rows: enough to fill the chip `over`
-// times, with at least two streamed tiles each, and up to four times while
-// they keep 32 tiles.  Twice over evens out the causal walks' lengths (dK/dV,
-// 4,096 tokens x 32/8 heads: 195 us against 250 at once over, 2,048 tokens 54
-// against 65); four times with 64-row waves, whose walks differ more (forward
-// 130 us against 141 and 187 at twice and once over, dQ 153 / 163 / 217), and
-// over long walks (8,192 tokens x 9/3 heads, forward 162 us against 186, dQ
-// 179 against 204), while short ones lose (2 x 2,047 tokens x 9/3 heads,
-// forward 48 us against 41).
+// Waves that share a block of stationary rows in dQ and dK/dV: enough to fill
+// the chip `over` times, with at least two streamed tiles each, and up to four
+// times while they keep 32 tiles.  Twice over evens out the causal walks'
+// lengths (dK/dV, 4,096 tokens x 32/8 heads: 195 us against 250 at once over,
+// 2,048 tokens 54 against 65); four times with 64-row waves, whose walks differ
+// more (dQ 153 us against 163 and 217 at twice and once over), and over long
+// walks (8,192 tokens x 9/3 heads, dQ 179 against 204).
 int split_for(int64_t blocks, int64_t tiles, int over) {
   int s = 1;
   while (s < 8 && tiles >= 4 * s &&
@@ -696,7 +694,9 @@ int split_for(int64_t blocks, int64_t tiles, int over) {
   return s;
 }
 
-// The same for the forward, whose short walks pay more for a further split (the
+// The same for the forward (where long walks gain alike: 4,096 tokens x 32/8 heads
+// 130 us at four times over against 141 and 187 at twice and once, 8,192 x 9/3
+// heads 162 against 186), whose short walks pay more for a further split (the
 // merge in LDS, a second round of workgroups) than they gain: within the waves
 // the chip holds while there are tiles for them (200 queries over 512 keys, 8 x
 // 16 heads: 14.3 us with two, 22.7 with eight; 100 queries over 64 keys, 8

@@ -20,12 +20,12 @@
 // with V^T from transposed LDS reads.
 //
 // Bound by the cache read once it is long (262,144 keys x 8 KV heads of 128:
-// 158 us + 5.5 us of merge, 6.6 TB/s) and by latency when it is short: a tile
-// takes 2 us to arrive, a workgroup 1 us to start.  Measured against the
-// blockwise forward that head_dim 64 and more than 16 rows took before (one
-// query call, caches cold): 4 sequences x 3,001 keys, 9/3 heads of 64
-// 69.9 -> 9.0 us; 8 tokens x 32/8 heads of 128 over 16,001 keys 266 -> 22.3 us;
-// 16 sequences x 60,000 keys of the same 1310 -> 730 us.  Against one-wave
+// 153-157 us + 5 us of merge, 6.8-7.0 TB/s) and by latency when it is short: a
+// tile takes 2 us to arrive, a workgroup 1 us to start.  Measured against the
+// blockwise forward that head_dim 64 and more than 16 rows took before (GPU
+// time of a call, caches cold): 4 sequences x 3,001 keys, 9/3 heads of 64
+// 70.9 -> 10.0 us; 8 tokens x 32/8 heads of 128 over 16,001 keys 272 -> 23.4 us;
+// 16 sequences x 60,000 keys of the same 1309 -> 726 us.  Against one-wave
 // workgroups with a merge for every shape: 8,001 keys x 32/8 heads
 // 15.2 -> 12.9 us, 16 x 4,000 66.7 -> 53 us.
 #include "common.h"
